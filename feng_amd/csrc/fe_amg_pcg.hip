@@ -2354,19 +2354,19 @@ int feAmgPcgPrepare(fe_hip_ctx *ctx)
   return FE_STATUS_OK;
 }
 
-int feAmgPcgVcycle(fe_hip_ctx *ctx, const double *r, double *z)
+void feAmgPcgNested(const fe_hip_ctx *ctx, const int **perm, double **rhs, const double **z)
+{
+  *perm = ctx->amgPcg->perm;
+  *rhs = ctx->amgPcg->rhs64v;
+  *z = ctx->amgPcg->z64v;
+}
+
+int feAmgPcgVcycleLaunch(fe_hip_ctx *ctx)
 {
   FE_REQUIRE(ctx, ctx->amgPcg, "nested multigrid: set up before the V-cycle");
   FeAmgPcg &A = *ctx->amgPcg;
-  FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the mailbox is written by the device
-  ((volatile PcgMailbox *)A.mbHost)->barErr = 0;
-  const bool val64 = !ctx->pcValues32;
-  const int n = A.lv[0].n;
-  const int gp = std::min(1024, (n + 255) / 256);
   PcgVecs<double> v = vecs64(A);
-  hipLaunchKernelGGL(pcgPermuteRhs<double>, dim3(gp), dim3(256), 0, ctx->stream, n, A.perm, r, v.rhs);
-  hipLaunchKernelGGL(pcgZero<double>, dim3(gp), dim3(256), 0, ctx->stream, n, v.x, A.done, A.stat);
-  if(val64) {
+  if(!ctx->pcValues32) {
     const PLev<double, double> L0 = pview<double, double>(A.lv[0]), L1 = pview<double, double>(A.lv[1]);
     hipLaunchKernelGGL((pcgDown0<double, double>), dim3(L0.nTiles), dim3(kFTB), 0, ctx->stream, L0, v.x,
                        (const double *)v.p[0], (const double *)v.q[0], (const double *)v.w, (const double *)v.rhs, v.r[0],
@@ -2381,6 +2381,22 @@ int feAmgPcgVcycle(fe_hip_ctx *ctx, const double *r, double *z)
                        A.done, A.stat, A.mbDev, 0, A.rr, A.bar);
     vcycleRest<double, float>(ctx, A, 1, v, v.r[0], v.u[0]);
   }
+  FE_HIP_TRY(ctx, hipGetLastError());
+  return FE_STATUS_OK;
+}
+
+int feAmgPcgVcycle(fe_hip_ctx *ctx, const double *r, double *z)
+{
+  FE_REQUIRE(ctx, ctx->amgPcg, "nested multigrid: set up before the V-cycle");
+  FeAmgPcg &A = *ctx->amgPcg;
+  FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the mailbox is written by the device
+  ((volatile PcgMailbox *)A.mbHost)->barErr = 0;
+  const int n = A.lv[0].n;
+  const int gp = std::min(1024, (n + 255) / 256);
+  PcgVecs<double> v = vecs64(A);
+  hipLaunchKernelGGL(pcgPermuteRhs<double>, dim3(gp), dim3(256), 0, ctx->stream, n, A.perm, r, v.rhs);
+  hipLaunchKernelGGL(pcgZero<double>, dim3(gp), dim3(256), 0, ctx->stream, n, v.x, A.done, A.stat);
+  if(int rc = feAmgPcgVcycleLaunch(ctx)) return rc;
   hipLaunchKernelGGL(pcgScatterBack<double>, dim3(gp), dim3(256), 0, ctx->stream, n, A.perm, (const double *)v.z, z);
   FE_HIP_TRY(ctx, hipGetLastError());
   FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));

@@ -31,6 +31,7 @@ struct FeFieldSplit {
   int nu = 0, np = 0;
   int64_t nnzF = 0;
   int *d_pOf = nullptr;    // unknown -> pressure index, -1 for the other unknowns
+  int *d_pRow = nullptr;   // pressure index -> unknown
   int *d_uRow = nullptr;   // velocity index -> unknown
   int *d_fmap = nullptr;   // entry of the velocity block (sub-context CSR) -> entry of A
   int *d_bia = nullptr, *d_bja = nullptr, *d_bmap = nullptr;  // A_up: velocity rows x pressure columns (CSR,
@@ -40,10 +41,15 @@ struct FeFieldSplit {
   int *d_sia = nullptr;    // per pressure row: its selfp terms
   int4 *d_sent = nullptr;  // (position of a_ik, of a_ki, of a_kk, 0), k a velocity unknown
   int *d_pDiag = nullptr;  // position of each pressure row's diagonal entry (-1: none)
-  double *d_sdinv = nullptr;
+  double *d_sdinv = nullptr;  // per unknown: 1 / S_kk of a pressure unknown
   double *d_ru = nullptr, *d_zu = nullptr;
+  // nested multigrid: per nested row of the velocity block its unknown and
+  // its row of A_up (d_bia, d_bja, d_bmap then follow the nested order), per
+  // unknown its nested row (-1: a pressure unknown)
+  int *d_nRow = nullptr, *d_nPos = nullptr;
   fe_hip_ctx *sub = nullptr;
-  bool nested = false;
+  bool nested = false, mapped = false;
+  std::vector<int> uRow, bia, bja, bmap;  // host copies until the order of A_up's rows is known
   double sign = 1.;  // -1 when the velocity block's diagonal is negative: its V-cycle runs on -A_uu
 };
 
@@ -59,8 +65,9 @@ __global__ void fsGather(int64_t cnt, const int *__restrict__ map, const double 
 }
 
 // 1 / diag(A_pp - A_pu diag(A_uu)^-1 A_up) per pressure row (1 where it is 0).
-__global__ void fsSchurDiag(int np, const int *__restrict__ sia, const int4 *__restrict__ sent,
-                            const double *__restrict__ val, const int *__restrict__ pDiag, double *__restrict__ sdinv)
+__global__ void fsSchurDiag(int np, const int *__restrict__ pRow, const int *__restrict__ sia,
+                            const int4 *__restrict__ sent, const double *__restrict__ val,
+                            const int *__restrict__ pDiag, double *__restrict__ sdinv)
 {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if(q >= np) return;
@@ -69,7 +76,7 @@ __global__ void fsSchurDiag(int np, const int *__restrict__ sia, const int4 *__r
     const int4 e = sent[t];
     s -= val[e.x] * val[e.y] / val[e.z];
   }
-  sdinv[q] = (s != 0. && s == s) ? 1. / s : 1.;
+  sdinv[pRow[q]] = (s != 0. && s == s) ? 1. / s : 1.;
 }
 
 // z_p = S^-1 r_p, z_u = 0.
@@ -78,8 +85,7 @@ __global__ void fsInit(int n, const int *__restrict__ pOf, const double *__restr
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
-  const int q = pOf[i];
-  z[i] = q >= 0 ? sdinv[q] * r[i] : 0.;
+  z[i] = pOf[i] >= 0 ? sdinv[i] * r[i] : 0.;
 }
 
 // ru = r_u - A_up z_p over the velocity rows (A_up with its own CSR: the
@@ -99,6 +105,40 @@ __global__ __launch_bounds__(256) void fsResidualU(int nu, const int *__restrict
 #pragma unroll
   for(int o = kFsLPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kFsLPR);
   if(on && sub == 0) ru[a] = r[i] - s;
+}
+
+// Nested multigrid: the right-hand side of the velocity block in its nested
+// order, rhs = r_u - A_up S^-1 r_p, S^-1 applied in the product (one launch
+// for z_p, the residual and the permutation).
+__global__ __launch_bounds__(256) void fsForward(int nu, const int *__restrict__ nRow, const int *__restrict__ bia,
+                                                 const int *__restrict__ bja, const double *__restrict__ bval,
+                                                 const double *__restrict__ sdinv, const double *__restrict__ r,
+                                                 double *__restrict__ rhs)
+{
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int a = t / kFsLPR, sub = t % kFsLPR;
+  const bool on = a < nu;
+  double s = 0., ri = 0.;
+  if(on) {
+    if(sub == 0) ri = r[nRow[a]];
+    for(int k = bia[a] + sub; k < bia[a + 1]; k += kFsLPR) {
+      const int j = bja[k];
+      s += bval[k] * (sdinv[j] * r[j]);
+    }
+  }
+#pragma unroll
+  for(int o = kFsLPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kFsLPR);
+  if(on && sub == 0) rhs[a] = ri - s;
+}
+
+// z over all unknowns: S^-1 r_p, and the V-cycle's result from its nested order.
+__global__ void fsBackward(int n, const int *__restrict__ nPos, const double *__restrict__ sdinv, double sign,
+                           const double *__restrict__ r, const double *__restrict__ zn, double *__restrict__ z)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i >= n) return;
+  const int p = nPos[i];
+  z[i] = p >= 0 ? sign * zn[p] : sdinv[i] * r[i];
 }
 
 __global__ void fsScatterU(int nu, const int *__restrict__ uRow, double sign, const double *__restrict__ zu,
@@ -214,12 +254,15 @@ int fsPattern(fe_hip_ctx *ctx)
     }
     sia[q + 1] = (int)sent.size();
   }
-  if(upload(ctx, &P.d_pOf, pOf) || upload(ctx, &P.d_uRow, uRow) || upload(ctx, &P.d_fmap, fmap) ||
-     upload(ctx, &P.d_sia, sia) || upload(ctx, &P.d_sent, sent) || upload(ctx, &P.d_pDiag, pDiag) ||
-     feAlloc(ctx, &P.d_sdinv, std::max(1, P.np)) || feAlloc(ctx, &P.d_ru, std::max(1, P.nu)) ||
-     feAlloc(ctx, &P.d_zu, std::max(1, P.nu)) || upload(ctx, &P.d_bia, bia) || upload(ctx, &P.d_bja, bja) ||
-     upload(ctx, &P.d_bmap, bmap) || feAlloc(ctx, &P.d_bval, std::max<int64_t>(1, P.nnzB)))
+  if(upload(ctx, &P.d_pOf, pOf) || upload(ctx, &P.d_pRow, pRow) || upload(ctx, &P.d_uRow, uRow) ||
+     upload(ctx, &P.d_fmap, fmap) || upload(ctx, &P.d_sia, sia) || upload(ctx, &P.d_sent, sent) ||
+     upload(ctx, &P.d_pDiag, pDiag) || feAlloc(ctx, &P.d_sdinv, std::max(1, n)) ||
+     feAlloc(ctx, &P.d_bval, std::max<int64_t>(1, P.nnzB)))
     return FE_STATUS_OUT_OF_MEMORY;
+  P.uRow.swap(uRow);
+  P.bia.swap(bia);
+  P.bja.swap(bja);
+  P.bmap.swap(bmap);
   // the velocity block's context: CSR of its own, the parent's stream, the
   // parent's multigrid settings
   fe_hip_ctx *sub = nullptr;
@@ -244,6 +287,39 @@ int fsPattern(fe_hip_ctx *ctx)
   return FE_STATUS_OK;
 }
 
+// Rows of A_up in the order the applications use (once per pattern): the
+// nested order of the velocity block, or its own order with the per-level
+// multigrid.
+int fsMaps(fe_hip_ctx *ctx)
+{
+  FeFieldSplit &P = *ctx->fieldSplit;
+  if(P.nested) {
+    const int *dperm = nullptr;
+    double *rhs = nullptr;
+    const double *zn = nullptr;
+    feAmgPcgNested(P.sub, &dperm, &rhs, &zn);
+    std::vector<int> perm(P.nu), nRow(P.nu), nPos(ctx->n, -1), nia(P.nu + 1, 0), nja, nmap;
+    FE_HIP_TRY(ctx, hipMemcpy(perm.data(), dperm, sizeof(int) * perm.size(), hipMemcpyDeviceToHost));
+    for(int p = 0; p < P.nu; ++p) {
+      const int a = perm[p];
+      nRow[p] = P.uRow[a];
+      nPos[P.uRow[a]] = p;
+      nja.insert(nja.end(), P.bja.begin() + P.bia[a], P.bja.begin() + P.bia[a + 1]);
+      nmap.insert(nmap.end(), P.bmap.begin() + P.bia[a], P.bmap.begin() + P.bia[a + 1]);
+      nia[p + 1] = (int)nja.size();
+    }
+    if(upload(ctx, &P.d_nRow, nRow) || upload(ctx, &P.d_nPos, nPos) || upload(ctx, &P.d_bia, nia) ||
+       upload(ctx, &P.d_bja, nja) || upload(ctx, &P.d_bmap, nmap))
+      return FE_STATUS_OUT_OF_MEMORY;
+  } else if(upload(ctx, &P.d_bia, P.bia) || upload(ctx, &P.d_bja, P.bja) || upload(ctx, &P.d_bmap, P.bmap) ||
+            feAlloc(ctx, &P.d_ru, std::max(1, P.nu)) || feAlloc(ctx, &P.d_zu, std::max(1, P.nu))) {
+    return FE_STATUS_OUT_OF_MEMORY;
+  }
+  P.mapped = true;
+  for(std::vector<int> *h : {&P.uRow, &P.bia, &P.bja, &P.bmap}) std::vector<int>().swap(*h);
+  return FE_STATUS_OK;
+}
+
 }  // namespace
 
 int feFieldSplitSetup(fe_hip_ctx *ctx)
@@ -257,11 +333,8 @@ int feFieldSplitSetup(fe_hip_ctx *ctx)
   if(P.nnzF > 0)
     hipLaunchKernelGGL(fsGather, dim3((unsigned)((P.nnzF + 255) / 256)), dim3(256), 0, ctx->stream, P.nnzF, P.d_fmap,
                        ctx->d_val, P.sign, sub->d_val);
-  if(P.nnzB > 0)
-    hipLaunchKernelGGL(fsGather, dim3((unsigned)((P.nnzB + 255) / 256)), dim3(256), 0, ctx->stream, P.nnzB, P.d_bmap,
-                       ctx->d_val, 1., P.d_bval);
   if(P.np > 0)
-    hipLaunchKernelGGL(fsSchurDiag, dim3((P.np + 255) / 256), dim3(256), 0, ctx->stream, P.np, P.d_sia, P.d_sent,
+    hipLaunchKernelGGL(fsSchurDiag, dim3((P.np + 255) / 256), dim3(256), 0, ctx->stream, P.np, P.d_pRow, P.d_sia, P.d_sent,
                        ctx->d_val, P.d_pDiag, P.d_sdinv);
   FE_HIP_TRY(ctx, hipGetLastError());
   if(int rc = feAmgSetup(sub)) {
@@ -274,6 +347,12 @@ int feFieldSplitSetup(fe_hip_ctx *ctx)
     ctx->setError("field split, velocity block: " + sub->err, __FILE__, __LINE__);
     return rc;
   }
+  if(!P.mapped)
+    if(int rcm = fsMaps(ctx)) return rcm;
+  if(P.nnzB > 0)
+    hipLaunchKernelGGL(fsGather, dim3((unsigned)((P.nnzB + 255) / 256)), dim3(256), 0, ctx->stream, P.nnzB, P.d_bmap,
+                       ctx->d_val, 1., P.d_bval);
+  FE_HIP_TRY(ctx, hipGetLastError());
   return FE_STATUS_OK;
 }
 
@@ -281,12 +360,27 @@ int feFieldSplitApply(fe_hip_ctx *ctx, const double *r, double *z)
 {
   FeFieldSplit &P = *ctx->fieldSplit;
   const int n = ctx->n;
+  if(P.nested) {
+    const int *perm = nullptr;
+    double *rhs = nullptr;
+    const double *zn = nullptr;
+    feAmgPcgNested(P.sub, &perm, &rhs, &zn);
+    hipLaunchKernelGGL(fsForward, dim3((unsigned)(((int64_t)P.nu * kFsLPR + 255) / 256)), dim3(256), 0, ctx->stream,
+                       P.nu, P.d_nRow, P.d_bia, P.d_bja, P.d_bval, P.d_sdinv, r, rhs);
+    if(int rc = feAmgPcgVcycleLaunch(P.sub)) {
+      ctx->setError("field split, velocity block: " + P.sub->err, __FILE__, __LINE__);
+      return rc;
+    }
+    hipLaunchKernelGGL(fsBackward, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, P.d_nPos, P.d_sdinv, P.sign, r,
+                       zn, z);
+    FE_HIP_TRY(ctx, hipGetLastError());
+    return FE_STATUS_OK;
+  }
   hipLaunchKernelGGL(fsInit, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, P.d_pOf, P.d_sdinv, r, z);
   if(P.nu > 0) {
     hipLaunchKernelGGL(fsResidualU, dim3((unsigned)(((int64_t)P.nu * kFsLPR + 255) / 256)), dim3(256), 0, ctx->stream,
                        P.nu, P.d_uRow, P.d_bia, P.d_bja, P.d_bval, z, r, P.d_ru);
-    const int rc = P.nested ? feAmgPcgVcycle(P.sub, P.d_ru, P.d_zu)
-                            : feAmgApply(P.sub, (const double *)P.d_ru, P.d_zu, nullptr, P.sub->pcValues32 != 0);
+    const int rc = feAmgApply(P.sub, (const double *)P.d_ru, P.d_zu, nullptr, P.sub->pcValues32 != 0);
     if(rc) {
       ctx->setError("field split, velocity block: " + P.sub->err, __FILE__, __LINE__);
       return rc;

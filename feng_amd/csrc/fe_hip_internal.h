@@ -178,6 +178,7 @@ struct FeMpnn;   // learned-preconditioner state (fe_learned.hip)
 struct FeAmg;    // aggregation multigrid hierarchy (fe_amg.hip)
 struct FeAmgPcg;  // nested-ordered multigrid PCG (fe_amg_pcg.hip)
 struct FeFieldSplit;  // Schur block preconditioner of saddle-point systems (fe_fieldsplit.hip)
+struct FeGmres;       // kept GMRES workspace (fe_gmres.hip)
 struct FeDirect;      // dense LU of the direct solve (fe_direct.hip)
 
 // Host copy of the aggregation hierarchy of the CSR pattern (built by
@@ -197,6 +198,7 @@ struct fe_hip_ctx {
   std::string err;
   FeFieldSplit *fieldSplit = nullptr;
   FeDirect *direct = nullptr;
+  FeGmres *gmres = nullptr;
 
   // mesh
   int dim = 0, V = 0, E = 0, nvpe = 0;
@@ -398,6 +400,7 @@ struct FeAmgPcgResult {
 int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out);
 int feSolveDirect(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_solve_stats *stats);
 void feDirectRelease(fe_hip_ctx *ctx);
+void feGmresRelease(fe_hip_ctx *ctx);
 int feAmgPcgSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double bnorm, double target, double *x64,
                   double *r64, FeAmgPcgResult *res);
 int feAmgPcgLevels(const fe_hip_ctx *ctx, int *levels, int *rows, int64_t *nnz, int cap);
@@ -414,6 +417,13 @@ int feAmgPcgFuseGrid(const fe_hip_ctx *ctx);  // workgroups of the fused coarse-
 int feAmgPcgApply(fe_hip_ctx *ctx, const double *r, double *z);
 int feAmgPcgPrepare(fe_hip_ctx *ctx);
 int feAmgPcgVcycle(fe_hip_ctx *ctx, const double *r, double *z);
+// The V-cycle in the nested order without copies or synchronization, for
+// callers that keep their own maps: the device permutation (nested row ->
+// row), the right-hand side it reads and the result it writes, and its
+// launches (feAmgPcgPrepare first; the fused coarse launch of amg_fuse, whose
+// barriers are checked after a synchronization, is not taken here).
+void feAmgPcgNested(const fe_hip_ctx *ctx, const int **perm, double **rhs, const double **z);
+int feAmgPcgVcycleLaunch(fe_hip_ctx *ctx);
 
 // Block upper-triangular Schur preconditioner of a saddle-point system
 // (fe_fieldsplit.hip): set-up of the current values, then z = P^-1 r on

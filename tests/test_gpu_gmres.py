@@ -1,0 +1,58 @@
+"""GMRES kept on the device (fe_gmres.hip): one to three rows' chunk of the dot
+products, cycle lengths around the 64-vector variant of the projection
+kernels and at the ends of the accepted range, both orthogonalizations,
+against dense solves; the iteration budget and the repeated solve."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(N):
+    from feng_amd.api import FN_CONST, TRI_P1, Fn, Mesh
+    from feng_amd.problems import advection_diffusion_system
+    one = Fn(FN_CONST, 1.0)
+    S, num = advection_diffusion_system(Mesh.square(N, 0.2, N), TRI_P1, 2, [Fn(FN_CONST, 30.0), Fn(FN_CONST, -20.0)], one,
+                                        Fn(FN_CONST, -1.0))
+    S.assemble(3)
+    ia, ja = S.get_csr()
+    val, rhs = S.get_system()
+    D = np.zeros((num.nInc, num.nInc))
+    D[np.repeat(np.arange(num.nInc), np.diff(ia)), ja] = val
+    return S, D, rhs
+
+
+@pytest.mark.parametrize("N", [2, 3, 24, 41])
+@pytest.mark.parametrize("restart", [2, 63, 64, 65, 120])
+def test_gmres_matches_dense_solve(N, restart):
+    from feng_amd.api import KSP_GMRES, PC_JACOBI
+    print("gmres", N, restart, flush=True)
+    S, D, rhs = _system(N)
+    x = np.linalg.solve(D, rhs)
+    # ||x - x*|| <= ||D^-1|| ||r||, ||r|| <= rtol ||b|| (and the rounding of the dense solve)
+    rtol = 1e-10
+    bound = np.linalg.norm(np.linalg.inv(D), 2) * 1.01 * rtol * np.linalg.norm(rhs)
+    for orth in (1, 2):
+        S.set_tuning("gmres_orth", orth)
+        r, du = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, rtol=rtol, restart=restart, max_iter=20000, want_du=True)
+        assert r.converged and r.reason == 2 and r.relres <= rtol
+        assert np.linalg.norm(du - x) <= bound
+        assert np.linalg.norm(rhs - D @ du) <= 1.01 * rtol * np.linalg.norm(rhs) + 1e-14 * np.linalg.norm(D) * np.linalg.norm(x)
+        assert abs(r.norm_dx_inf - np.abs(du).max()) <= 1e-15 * np.abs(du).max()
+        assert r.norm_rhs_inf == np.abs(rhs).max()
+        again, du2 = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, rtol=rtol, restart=restart, max_iter=20000, want_du=True)
+        assert again.iterations == r.iterations and np.array_equal(du, du2)  # bitwise repeatable
+    S.close()
+
+
+def test_gmres_iteration_budget_and_zero_rhs():
+    from feng_amd.api import KSP_GMRES, PC_JACOBI
+    S, D, rhs = _system(24)
+    for restart, most in ((50, 7), (4, 4), (4, 6), (50, 0)):
+        r, du = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, rtol=1e-12, restart=restart, max_iter=most, want_du=True)
+        assert not r.converged and r.reason == -3 and r.iterations == most
+        assert abs(r.relres - np.linalg.norm(rhs - D @ du) / np.linalg.norm(rhs)) <= 1e-10
+    S.set_system(rhs=np.zeros_like(rhs))
+    r, du = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, rtol=1e-12, want_du=True)
+    assert r.converged and r.iterations == 0 and not du.any()
+    S.close()

@@ -482,6 +482,7 @@ struct Gm {
     }
     if(pc == FE_PC_FIELDSPLIT) return feFieldSplitApply(ctx, v, out);
     FePrecond &P = ctx->pc;
+    if(sweeps == 0 && feTriSolveUsable(ctx)) return feTriSolveApply(ctx, v, out);
     if(sweeps == 0) {
       // exact: y = L^-1 v (G_L = I - L_strict: y_i = v_i + sum_j<i g_ij y_j), then
       // z = U^-1 y (z_i = y_i / u_ii + sum_j>i g_ij z_j with g_ij = -u_ij / u_ii)
@@ -669,6 +670,11 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
   ctx->iterTimer = FeKernelTimer{std::move(ctx->iterTimer.ev)};
   if(g.pc == FE_PC_ILU0) {
     if(int rc = fePrecondFactor(ctx)) return rc;
+    if(g.sweeps == 0) {
+      if(int rc = feTriSolveBuild(ctx)) return rc;
+      if(feTriSolveUsable(ctx))
+        if(int rc = feTriSolvePack(ctx)) return rc;
+    }
   } else if(g.pc == FE_PC_FIELDSPLIT) {
     if(int rc = feFieldSplitSetup(ctx)) return rc;
   } else if(g.pc == FE_PC_JACOBI) {

@@ -178,6 +178,7 @@ struct FeMpnn;   // learned-preconditioner state (fe_learned.hip)
 struct FeAmg;    // aggregation multigrid hierarchy (fe_amg.hip)
 struct FeAmgPcg;  // nested-ordered multigrid PCG (fe_amg_pcg.hip)
 struct FeFieldSplit;  // Schur block preconditioner of saddle-point systems (fe_fieldsplit.hip)
+struct FeTriSolve;    // one-launch exact ILU(0) application (fe_trisolve.hip)
 struct FeGmres;       // kept GMRES workspace (fe_gmres.hip)
 struct FeDirect;      // dense LU of the direct solve (fe_direct.hip)
 
@@ -199,6 +200,7 @@ struct fe_hip_ctx {
   FeFieldSplit *fieldSplit = nullptr;
   FeDirect *direct = nullptr;
   FeGmres *gmres = nullptr;
+  FeTriSolve *tri = nullptr;
 
   // mesh
   int dim = 0, V = 0, E = 0, nvpe = 0;
@@ -401,6 +403,14 @@ int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out);
 int feSolveDirect(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_solve_stats *stats);
 void feDirectRelease(fe_hip_ctx *ctx);
 void feGmresRelease(fe_hip_ctx *ctx);
+// Exact ILU(0) application in one launch (fe_trisolve.hip): the schedule
+// (once per pattern, after fePrecondFactor), the values of the last
+// factorization, z = U^-1 L^-1 v on device vectors.
+int feTriSolveBuild(fe_hip_ctx *ctx);
+bool feTriSolveUsable(const fe_hip_ctx *ctx);
+int feTriSolvePack(fe_hip_ctx *ctx);
+int feTriSolveApply(fe_hip_ctx *ctx, const double *v, double *z);
+void feTriSolveRelease(fe_hip_ctx *ctx);
 int feAmgPcgSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double bnorm, double target, double *x64,
                   double *r64, FeAmgPcgResult *res);
 int feAmgPcgLevels(const fe_hip_ctx *ctx, int *levels, int *rows, int64_t *nnz, int cap);

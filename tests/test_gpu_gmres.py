@@ -56,3 +56,33 @@ def test_gmres_iteration_budget_and_zero_rhs():
     r, du = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, rtol=1e-12, want_du=True)
     assert r.converged and r.iterations == 0 and not du.any()
     S.close()
+
+
+@pytest.mark.parametrize("kind, N", [(1, 2), (1, 9), (2, 20), (5, 7), (6, 6), (3, 6), (1, 129), (1, 130)])
+def test_exact_ilu0_application(kind, N):
+    """One GMRES step from x = 0 returns a multiple of U^-1 L^-1 b: the exact
+    application of the factor against host triangular solves, one unknown to
+    the largest vector of the one-launch schedule (16,384) and past it."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as sl
+    from feng_amd.api import FN_CONST, KSP_GMRES, PC_ILU0, Fn, Mesh
+    from feng_amd.problems import advection_diffusion_system, navier_stokes_system
+    print("ilu0 application", kind, N, flush=True)
+    m = Mesh.square(N, 0.2, N)
+    if kind == 3:  # Taylor-Hood: rows of two fields
+        S, num = navier_stokes_system(m, 40.0, 5)
+    else:
+        S, num = advection_diffusion_system(m, kind, 4, [Fn(FN_CONST, 5.0), Fn(FN_CONST, -3.0)], Fn(FN_CONST, 1.0),
+                                            Fn(FN_CONST, -1.0))
+    S.assemble(3)
+    b = np.random.default_rng(N).normal(size=num.nInc)
+    S.set_system(rhs=b)
+    r, du = S.solve(ksp=KSP_GMRES, pc=PC_ILU0, rtol=1e-14, restart=2, max_iter=1, want_du=True)
+    ia, ja = S.get_csr()
+    lu = sp.csr_matrix((S.get_factor(), ja, ia), shape=(num.nInc, num.nInc))
+    y = sl.spsolve_triangular((sp.tril(lu, -1) + sp.identity(num.nInc)).tocsr(), b, lower=True)
+    z = sl.spsolve_triangular(sp.triu(lu).tocsr(), y, lower=False)
+    t = du @ z / (z @ z)
+    # rounding of the solves only: (longest row + levels) units in the last place, amplified by the growth in z
+    assert np.linalg.norm(du - t * z) <= 1e-10 * np.linalg.norm(du)
+    S.close()

@@ -274,6 +274,7 @@ int fe_hip_ctx_destroy(fe_hip_ctx *ctx)
   feDirectRelease(ctx);
   feGmresRelease(ctx);
   feTriSolveRelease(ctx);
+  feResidentRelease(ctx);
   for(void *p : ctx->owned) (void)hipFree(p);
   for(auto &g : ctx->graphs) (void)hipGraphExecDestroy((hipGraphExec_t)g.second);
   ctx->graphs.clear();
@@ -749,6 +750,9 @@ int fe_hip_set_tuning(fe_hip_ctx *ctx, const char *key, int value)
   } else if(k == "gmres_orth") {
     FE_REQUIRE(ctx, value == 1 || value == 2, "gmres_orth must be 1 (classical Gram-Schmidt) or 2 (CGS2)");
     ctx->gmresOrth = value;
+  } else if(k == "resident") {
+    FE_REQUIRE(ctx, value == 0 || value == 1, "resident must be 0 or 1");
+    ctx->resident = value;
   } else if(k == "ilu_sweeps") {
     FE_REQUIRE(ctx, value >= 0 && value <= 64,
                "ilu_sweeps must be 0 (exact triangular solves) or a sweep count in [1, 64]");
@@ -843,6 +847,7 @@ int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value)
   else if(k == "pipe_kernel") *value = ctx->pipeKernel;
   else if(k == "ic0_sweeps") *value = ctx->icSweeps;
   else if(k == "ilu_sweeps") *value = ctx->pc.sweeps;
+  else if(k == "resident") *value = ctx->resident;
   else if(k == "gmres_orth") *value = ctx->gmresOrth;
   else if(k == "pc_fp32") *value = ctx->pcFp32;
   else if(k == "pc_values32") *value = ctx->pcValues32;

@@ -179,6 +179,7 @@ struct FeAmg;    // aggregation multigrid hierarchy (fe_amg.hip)
 struct FeAmgPcg;  // nested-ordered multigrid PCG (fe_amg_pcg.hip)
 struct FeFieldSplit;  // Schur block preconditioner of saddle-point systems (fe_fieldsplit.hip)
 struct FeTriSolve;    // one-launch exact ILU(0) application (fe_trisolve.hip)
+struct FeResident;    // all-iterations-in-one-launch Jacobi-PCG (fe_resident.hip)
 struct FeGmres;       // kept GMRES workspace (fe_gmres.hip)
 struct FeDirect;      // dense LU of the direct solve (fe_direct.hip)
 
@@ -201,6 +202,9 @@ struct fe_hip_ctx {
   FeDirect *direct = nullptr;
   FeGmres *gmres = nullptr;
   FeTriSolve *tri = nullptr;
+  FeResident *res = nullptr;
+  int resident = 1;             // FP64 Jacobi-PCG: all iterations in one launch where the system fits (0: never)
+  bool residentGaveUp = false;  // a wait of a resident launch ran out: this context keeps the other kernels
 
   // mesh
   int dim = 0, V = 0, E = 0, nvpe = 0;
@@ -411,6 +415,17 @@ bool feTriSolveUsable(const fe_hip_ctx *ctx);
 int feTriSolvePack(fe_hip_ctx *ctx);
 int feTriSolveApply(fe_hip_ctx *ctx, const double *v, double *z);
 void feTriSolveRelease(fe_hip_ctx *ctx);
+// FP64 Jacobi-PCG of A x = rhs with all iterations, the checks of the true
+// residual and the restarts in one launch (fe_resident.hip).  ran = false: the
+// system does not fit the kernel (or a wait gave up) and the caller solves
+// with its own kernels.
+struct FeResidentResult {
+  bool ran;
+  int reason, iters, outer;
+  double relres, inf[3];  // inf: ||x||, ||rhs||, ||rhs - A x||
+};
+int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res);
+void feResidentRelease(fe_hip_ctx *ctx);
 int feAmgPcgSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double bnorm, double target, double *x64,
                   double *r64, FeAmgPcgResult *res);
 int feAmgPcgLevels(const fe_hip_ctx *ctx, int *levels, int *rows, int64_t *nnz, int cap);

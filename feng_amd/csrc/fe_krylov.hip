@@ -1727,6 +1727,38 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_sol
   ctx->iterTimer.total_ms = 0.;
   ctx->iterTimer.launches = 0;
 
+  // FP64 Jacobi-PCG: the same recurrences with the whole solve in one launch,
+  // where the system fits
+  if(!split && o->precision == FE_PREC_FP64 && tiled64) {
+    FeResidentResult R;
+    if(int rc = feResidentJacobi(ctx, o, ctx->d_du, &R)) return rc;
+    if(R.ran) {
+      FE_HIP_TRY(ctx, hipEventRecord(t1, ctx->stream));
+      FE_HIP_TRY(ctx, hipEventSynchronize(t1));
+      float ms = 0.f;
+      FE_HIP_TRY(ctx, hipEventElapsedTime(&ms, t0, t1));
+      (void)hipEventDestroy(t0);
+      (void)hipEventDestroy(t1);
+      if(stats) {
+        memset(stats, 0, sizeof(*stats));
+        stats->iterations = R.iters;
+        stats->outer_iterations = R.outer;
+        stats->converged = R.reason > 0 ? 1 : 0;
+        stats->reason = R.reason;
+        stats->relres_fp64 = R.relres;
+        stats->norm_dx_inf = R.inf[0];
+        stats->norm_rhs_inf = R.inf[1];
+        stats->norm_axb_inf = R.inf[2];
+        stats->ms_solve = ms;
+      }
+      if(du) {
+        FE_HIP_TRY(ctx, hipMemcpyAsync(du, ctx->d_du, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
+        FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+      }
+      return FE_STATUS_OK;
+    }
+  }
+
   hipLaunchKernelGGL(sumSquares, dim3(kGrid), dim3(kTB), 0, ctx->stream, n, ctx->d_rhs, w.part);
   hipLaunchKernelGGL(finalizeSums, dim3(1), dim3(kTB), 0, ctx->stream, w.part, kGrid, 1, w.res + 8);
   FE_HIP_TRY(ctx, hipGetLastError());

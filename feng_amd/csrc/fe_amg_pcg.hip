@@ -37,7 +37,7 @@
 // the FP64 residual replaces the recursive one and the stopped iteration is
 // redone from the kept search direction (no restart, the Krylov history
 // carries over).
-#include "fe_hip_internal.h"
+#include "fe_amg_nested.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1949,7 +1949,8 @@ int pcgNumeric(fe_hip_ctx *ctx, bool fp64Values, bool fp64Product, int slot)
     hipLaunchKernelGGL(pcgWDenseInverse, dim3(1), dim3(1024), 0, ctx->stream, Dl.n, (const int *)Dl.ia,
                        (const int *)Dl.ja, (const double *)Dl.val64, (float *)(A.wImg + W.oDinv - W.oImg), A.flag);
   }
-  // the static LDS image of the small-level kernel for this slot
+  // the static LDS image of the small-level kernel for this slot (slot < 0: none)
+  if(slot < 0) return FE_STATUS_OK;
   const PBlockPlan &pl = A.plan[slot];
   if(slot == 0)
     hipLaunchKernelGGL((pcgPackBlock<float, float>), dim3(1), dim3(kPBlockTB), 0, ctx->stream,
@@ -2351,6 +2352,20 @@ int feAmgPcgPrepare(fe_hip_ctx *ctx)
   FE_HIP_TRY(ctx, hipMemcpyAsync(&flag, A.flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   FE_REQUIRE(ctx, flag == 0, "AMG: the coarsest operator is not positive definite");
+  return FE_STATUS_OK;
+}
+
+int feAmgNestedPrepare(fe_hip_ctx *ctx, FeNestedView *view)
+{
+  if(!ctx->amgPcg)
+    if(int rc = pcgSetupPattern(ctx)) return rc;
+  if(int rc = pcgNumeric(ctx, false, true, -1)) return rc;
+  const FeAmgPcg &A = *ctx->amgPcg;
+  for(const FeAmgPcgLevel &h : A.lv)
+    view->lv.push_back(FeNestedLevel{h.n, h.nc, h.nnz, h.sell, h.ia, h.ja, h.agg, h.aggStart, h.valD, h.val32, h.l1_32});
+  view->perm = A.perm;
+  view->cinv = A.cinv64;
+  view->flag = A.flag;
   return FE_STATUS_OK;
 }
 

@@ -275,6 +275,7 @@ int fe_hip_ctx_destroy(fe_hip_ctx *ctx)
   feGmresRelease(ctx);
   feTriSolveRelease(ctx);
   feResidentRelease(ctx);
+  feAmgResidentRelease(ctx);
   for(void *p : ctx->owned) (void)hipFree(p);
   for(auto &g : ctx->graphs) (void)hipGraphExecDestroy((hipGraphExec_t)g.second);
   ctx->graphs.clear();

@@ -180,6 +180,7 @@ struct FeAmgPcg;  // nested-ordered multigrid PCG (fe_amg_pcg.hip)
 struct FeFieldSplit;  // Schur block preconditioner of saddle-point systems (fe_fieldsplit.hip)
 struct FeTriSolve;    // one-launch exact ILU(0) application (fe_trisolve.hip)
 struct FeResident;    // all-iterations-in-one-launch Jacobi-PCG (fe_resident.hip)
+struct FeAmgResident; // all-iterations-in-one-launch multigrid PCG (fe_amg_resident.hip)
 struct FeGmres;       // kept GMRES workspace (fe_gmres.hip)
 struct FeDirect;      // dense LU of the direct solve (fe_direct.hip)
 
@@ -203,7 +204,8 @@ struct fe_hip_ctx {
   FeGmres *gmres = nullptr;
   FeTriSolve *tri = nullptr;
   FeResident *res = nullptr;
-  int resident = 1;             // FP64 Jacobi-PCG: all iterations in one launch where the system fits (0: never)
+  FeAmgResident *amgRes = nullptr;
+  int resident = 1;             // FP64 Jacobi- and multigrid-PCG: all iterations in one launch where the system fits (0: never)
   bool residentGaveUp = false;  // a wait of a resident launch ran out: this context keeps the other kernels
 
   // mesh
@@ -426,6 +428,11 @@ struct FeResidentResult {
 };
 int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res);
 void feResidentRelease(fe_hip_ctx *ctx);
+// The same for the nested-ordered multigrid PCG with FP64 vectors and FP32
+// level values (fe_amg_resident.hip), numeric set-up included; after
+// feAmgSetup, where feAmgNestedUsable.
+int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res);
+void feAmgResidentRelease(fe_hip_ctx *ctx);
 int feAmgPcgSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double bnorm, double target, double *x64,
                   double *r64, FeAmgPcgResult *res);
 int feAmgPcgLevels(const fe_hip_ctx *ctx, int *levels, int *rows, int64_t *nnz, int cap);

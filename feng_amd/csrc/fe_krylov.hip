@@ -1727,11 +1727,18 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_sol
   ctx->iterTimer.total_ms = 0.;
   ctx->iterTimer.launches = 0;
 
-  // FP64 Jacobi-PCG: the same recurrences with the whole solve in one launch,
-  // where the system fits
-  if(!split && o->precision == FE_PREC_FP64 && tiled64) {
+  // FP64 Jacobi- and multigrid-PCG: the same methods with the whole solve in
+  // one launch, where the system fits
+  if(((!split && tiled64) || amg) && o->precision == FE_PREC_FP64) {
     FeResidentResult R;
-    if(int rc = feResidentJacobi(ctx, o, ctx->d_du, &R)) return rc;
+    R.ran = false;
+    if(!amg) {
+      if(int rc = feResidentJacobi(ctx, o, ctx->d_du, &R)) return rc;
+    } else {
+      if(int rc = feAmgSetup(ctx)) return rc;
+      if(feAmgNestedUsable(ctx))
+        if(int rc = feAmgResidentSolve(ctx, o, ctx->d_du, &R)) return rc;
+    }
     if(R.ran) {
       FE_HIP_TRY(ctx, hipEventRecord(t1, ctx->stream));
       FE_HIP_TRY(ctx, hipEventSynchronize(t1));

@@ -24,6 +24,11 @@
 
 #include "fe_hip_internal.h"
 
+#include <mutex>
+
+// Held from a resident launch to its end (one per device).
+std::mutex &feResidentMutex(int device);
+
 namespace fe_res {
 
 constexpr unsigned long long kSentinel = 0x7FF4DEAD5EA7F00Dull;

@@ -337,6 +337,7 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
     double y = 0.;
 #pragma unroll
     for(int e = 0; e < E / 2; ++e) {
+      asm volatile("" : "+v"(ix[e]));  // unpacked here, not kept unpacked across the loop
       y += v[2 * e] * reg[ix[e] & 0xffffu];
       y += v[2 * e + 1] * reg[ix[e] >> 16];
     }

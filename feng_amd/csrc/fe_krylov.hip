@@ -1692,6 +1692,8 @@ __global__ void castResidual(int n, const double *__restrict__ a, T *__restrict_
 
 }  // namespace
 
+constexpr int kAmgFp32From = 700000;
+
 int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out)
 {
   Workspace w;
@@ -1699,8 +1701,9 @@ int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out)
   return residualNorm2(ctx, w, x, ctx->d_rhs, r, out);
 }
 
-int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_solve_stats *stats)
+int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip_solve_stats *stats)
 {
+  const fe_hip_solver_opts *o = given;
   if(o->ksp == FE_KSP_GMRES) return feSolveGmres(ctx, o, du, stats);
   if(o->ksp == FE_KSP_DIRECT) return feSolveDirect(ctx, o, du, stats);
   FE_REQUIRE(ctx, o->ksp == FE_KSP_CG, "unknown Krylov method");
@@ -1709,6 +1712,21 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hip_sol
   const bool split = (o->pc != FE_PC_JACOBI);
   const bool amg = (o->pc == FE_PC_AMG);
   ctx->amgActive = amg;
+  // Multigrid-PCG with FP32 inner solves (FE_PREC_FP32_IR), up to kAmgFp32From
+  // rows: the FP64 iteration (level values stay FP32) instead.  A launch or a
+  // wait costs the same in either precision, and an FP32 product needs a
+  // restart or a replaced residual each time the residual has fallen by
+  // inner_rtol.  Solve, FP32 -> FP64, nested kernels: P2 triangles, 588,289
+  // rows, 1e4 contrast 80 -> 41 ms (647 -> 259 iterations), 576,081 rows,
+  // constant 32.8 -> 15.2 ms; P1 triangles, 488,601 rows 9.3 -> 8.4 ms; P1
+  // tetrahedra, 421,875 rows 7.2 -> 6.8 ms, level at 704,969 rows (10.9 and
+  // 11.1 ms), above which bytes decide.  Per-level kernels: P1 tetrahedra,
+  // 493,039 rows 26.1 -> 14.8 ms; P2 triangles, 249,001 rows 68.5 -> 49.5 ms.
+  fe_hip_solver_opts wide = *given;
+  if(amg && given->precision == FE_PREC_FP32_IR && ctx->pcValues32 && ctx->n <= kAmgFp32From) {
+    wide.precision = FE_PREC_FP64;
+    o = &wide;
+  }
   // pipelined form per precision: the tiled Ghysels-Vanroose iteration (one
   // gathered vector) for FP64 solves, Chronopoulos-Gear (w = A u every
   // iteration, fewer refinement restarts) for FP32 inner solves

@@ -99,7 +99,7 @@ typedef struct {
 #define FE_PC_FIELDSPLIT 7
 
 #define FE_PREC_FP64 0    /* FP64 Krylov */
-#define FE_PREC_FP32_IR 1 /* FP32 inner Krylov + FP64 iterative refinement */
+#define FE_PREC_FP32_IR 1 /* FP32 inner Krylov + FP64 iterative refinement (multigrid-PCG: FP64 up to 700,000 rows) */
 
 typedef struct {
   int ksp;           /* FE_KSP_* */

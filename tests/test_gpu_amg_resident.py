@@ -76,3 +76,22 @@ def test_resident_amg_high_contrast_and_floor():
             assert r1.converged and r1.relres <= rtol
         assert np.linalg.norm(x1 - x0) <= 1e-6 * np.linalg.norm(x0)
     S.close()
+
+
+@pytest.mark.parametrize("kernel,resident", [(2, 1), (2, 0), (1, 1)])
+def test_fp32_multigrid_runs_the_fp64_iteration(kernel, resident):
+    """Up to 700,000 rows FP32_IR multigrid-PCG is the FP64 iteration: the same
+    iterates bit for bit, from an FP32 assembly as from an FP64 one."""
+    from feng_amd.api import PC_AMG, PREC_FP32_IR, PREC_FP64
+    S, num = _system(4, 9)
+    S.set_tuning("amg_kernel", kernel)
+    S.set_tuning("resident", resident)
+    out = {}
+    for prec in (PREC_FP64, PREC_FP32_IR):
+        S.setToZero()
+        S.assemble(3, prec)
+        out[prec] = S.solve(pc=PC_AMG, precision=prec, rtol=1e-8, inner_rtol=1e-3, want_du=True)
+    (r0, d0), (r1, d1) = out[PREC_FP64], out[PREC_FP32_IR]
+    assert r0.converged and r1.iterations == r0.iterations and r1.outer_iterations == r0.outer_iterations
+    assert np.array_equal(d0, d1)
+    S.close()

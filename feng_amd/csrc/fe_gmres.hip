@@ -682,6 +682,11 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
   }
   FE_HIP_TRY(ctx, hipEventRecord(ev[1], ctx->stream));
 
+  // Level-scheduled exact solves (hundreds of launches) hide the host's round
+  // trip by themselves, and a step launched past a stop costs another
+  // application: cycles of one or two steps, as at the FP64 floor of a system
+  // (P4 triangles, n = 16,129), took 12 ms a step with kGmAhead, 8 with one.
+  const unsigned long long ahead = g.pc == FE_PC_ILU0 && g.sweeps == 0 && !feTriSolveUsable(ctx) ? 1 : kGmAhead;
   const int gNext = 1 + std::min(kG, (n + kTB - 1) / kTB);
   int iters = 0, outer = 0, converged = 0, reason = 0;
   unsigned long long step = 0;  // posted steps: one per cycle start and per Arnoldi step
@@ -702,8 +707,8 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
     const unsigned long long base = step;
     int j = 0, jn = 0;
     for(; !(word & 3) && !last && j < m && iters + j < o->max_iter; ++j) {
-      if(step >= kGmAhead) {
-        word = g.waitFor(step - kGmAhead + 1);
+      if(step >= ahead) {
+        word = g.waitFor(step - ahead + 1);
         if(word & 3) break;
       }
       double *vj = g.V + g.ld * j, *hcol = g.H + (size_t)j * ldh;

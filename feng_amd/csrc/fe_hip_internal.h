@@ -427,6 +427,8 @@ struct FeResidentResult {
   double relres, inf[3];  // inf: ||x||, ||rhs||, ||rhs - A x||
 };
 int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res);
+// Split-preconditioned PCG (IC(0), learned) the same way, factor set up before.
+int feResidentSplit(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res);
 void feResidentRelease(fe_hip_ctx *ctx);
 // The same for the nested-ordered multigrid PCG with FP64 vectors and FP32
 // level values (fe_amg_resident.hip), numeric set-up included; after

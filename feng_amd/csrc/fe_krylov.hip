@@ -1723,7 +1723,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   // 11.1 ms), above which bytes decide.  Per-level kernels: P1 tetrahedra,
   // 493,039 rows 26.1 -> 14.8 ms; P2 triangles, 249,001 rows 68.5 -> 49.5 ms.
   fe_hip_solver_opts wide = *given;
-  if(amg && given->precision == FE_PREC_FP32_IR && ctx->pcValues32 && ctx->n <= kAmgFp32From) {
+  if(amg && given->precision == FE_PREC_FP32_IR && ctx->d_val32 && ctx->pcValues32 && ctx->n <= kAmgFp32From) {
     wide.precision = FE_PREC_FP64;
     o = &wide;
   }
@@ -1745,9 +1745,14 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   ctx->iterTimer.total_ms = 0.;
   ctx->iterTimer.launches = 0;
 
-  // FP64 Jacobi- and multigrid-PCG: the same methods with the whole solve in
-  // one launch, where the system fits
-  if(((!split && tiled64) || amg) && o->precision == FE_PREC_FP64) {
+  // Jacobi- and multigrid-PCG with the whole solve in one launch, where the
+  // system fits; the split preconditioners follow their set-up.  FP32 inner
+  // solves (FE_PREC_FP32_IR) take the FP64 launch too: exchanges bound it, and
+  // restarts from the true residual cost iterations.  Jacobi, P1 tetrahedra
+  // 64^3: FP32 11.6 ms (552 iterations), here 2.7 (422); learned factor 45^3:
+  // 5.7 ms (162), here 1.7 (121).
+  if((!split && tiled64 && (o->precision == FE_PREC_FP64 || ctx->d_val32)) ||
+     (amg && o->precision == FE_PREC_FP64)) {
     FeResidentResult R;
     R.ran = false;
     if(!amg) {
@@ -1825,12 +1830,21 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
     w.s64.iaU = w.s32.iaU = P.d_iaU; w.s64.jaU = w.s32.jaU = P.d_jaU;
   }
 
+  FeResidentResult one{};
+  if(split && !amg && bn != 0. && (o->precision == FE_PREC_FP64 || ctx->d_val32))
+    if(int rc = feResidentSplit(ctx, o, ctx->d_du, &one)) return rc;
   const bool nested = amg && feAmgNestedUsable(ctx);
   if(bn == 0.) {
     FE_HIP_TRY(ctx, hipMemsetAsync(ctx->d_du, 0, sizeof(double) * n, ctx->stream));
     converged = 1;
     reason = 2;
     relres = 0.;
+  } else if(one.ran) {  // the whole solve in one launch
+    iters = one.iters;
+    outer = one.outer;
+    reason = one.reason;
+    converged = reason > 0 ? 1 : 0;
+    relres = one.relres;
   } else if(nested) {
     // multigrid PCG over the nested ordering, FP32 or FP64 inner solves under
     // FP64 refinement (fe_amg_pcg.hip)
@@ -2015,15 +2029,17 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
 
   if(stats) {
     memset(stats, 0, sizeof(*stats));
-    double dummy = 0.;
-    if(int rc = residualNorm2(ctx, w, ctx->d_du, ctx->d_rhs, w.tmp64, &dummy)) return rc;
-    hipLaunchKernelGGL(blockMaxAbs3, dim3(kGrid), dim3(kTB), 0, ctx->stream, n, ctx->d_du, ctx->d_rhs, w.tmp64,
-                       w.part);
-    hipLaunchKernelGGL(finalizeMax, dim3(1), dim3(64), 0, ctx->stream, w.part, kGrid, 3, w.res + 16);
-    FE_HIP_TRY(ctx, hipGetLastError());
-    double inf[3];
-    FE_HIP_TRY(ctx, hipMemcpyAsync(inf, w.res + 16, sizeof(inf), hipMemcpyDeviceToHost, ctx->stream));
-    FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    double inf[3] = {one.inf[0], one.inf[1], one.inf[2]};
+    if(!one.ran) {
+      double dummy = 0.;
+      if(int rc = residualNorm2(ctx, w, ctx->d_du, ctx->d_rhs, w.tmp64, &dummy)) return rc;
+      hipLaunchKernelGGL(blockMaxAbs3, dim3(kGrid), dim3(kTB), 0, ctx->stream, n, ctx->d_du, ctx->d_rhs, w.tmp64,
+                         w.part);
+      hipLaunchKernelGGL(finalizeMax, dim3(1), dim3(64), 0, ctx->stream, w.part, kGrid, 3, w.res + 16);
+      FE_HIP_TRY(ctx, hipGetLastError());
+      FE_HIP_TRY(ctx, hipMemcpyAsync(inf, w.res + 16, sizeof(inf), hipMemcpyDeviceToHost, ctx->stream));
+      FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    }
     stats->iterations = iters;
     stats->outer_iterations = outer;
     stats->converged = converged;

@@ -1,7 +1,8 @@
-// Jacobi-PCG with all iterations in one launch (the KSPCG / PCJACOBI of the
-// reference's options, feLinearSystemPETSc.cpp:900-1031): the pipelined
-// recurrences of fe_krylov.hip's tileIter (Ghysels & Vanroose 2014), with the
-// matrix in registers.
+// Jacobi-PCG, and split-preconditioned PCG (resSplit), with all iterations in
+// one launch (the KSPCG / PCJACOBI of the reference's options,
+// feLinearSystemPETSc.cpp:900-1031): the pipelined recurrences of
+// fe_krylov.hip's tileIter (Ghysels & Vanroose 2014), with the matrix in
+// registers.
 //
 // What bounded the launch-per-iteration form below some 10^5 unknowns was not
 // the matrix but the chain inside a launch -- dispatch, row bounds, columns
@@ -30,6 +31,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 using namespace fe_res;
@@ -48,6 +50,9 @@ struct FeResident {
   int *d_hcol = nullptr, *d_hcnt = nullptr;
   unsigned long long *d_buf = nullptr;  // kResBufs x (n values, 3 G partial sums)
   ResOut *d_out = nullptr, *h_out = nullptr;  // h_out: pinned copy
+  int splitState = 0;             // split PCG: 1 ready, -1 the factor's pattern is not the matrix's
+  int *d_pos = nullptr;
+  unsigned long long *d_splitBuf = nullptr;
 };
 
 namespace {
@@ -152,6 +157,26 @@ __global__ void resFill(size_t count, unsigned long long *__restrict__ buf, ResO
   for(size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
     buf[i] = kSentinel;
   if(blockIdx.x == 0 && threadIdx.x == 0) *out = ResOut{0, 0, 0, 0, 0., 0.};
+}
+
+// The workgroup's largest |x|, |b|, |b - A x|.
+template <int TB>
+__device__ __forceinline__ void resMaxima(bool own, double x, double b, double r, double (&part)[3][TB / 64], double *out)
+{
+  const int t = threadIdx.x;
+  double mx[3] = {own ? fabs(x) : 0., fabs(b), own ? fabs(r) : 0.};
+#pragma unroll
+  for(int k = 0; k < 3; ++k) {
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1) mx[k] = fmax(mx[k], __shfl_xor(mx[k], o, 64));
+    if((t & 63) == 0) part[k][t >> 6] = mx[k];
+  }
+  resBarrier();
+  if(t < 3) {
+    double mm = 0.;
+    for(int k = 0; k < TB / 64; ++k) mm = fmax(mm, part[t][k]);
+    out[t] = mm;
+  }
 }
 
 // What the values gathered by an exchange are, and its partial sums: the
@@ -378,26 +403,322 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
     }
   }
   if(own) a.x[row] = x;
-  // the workgroup's largest |x|, |b|, |b - A x|
-  double mx[3] = {own ? fabs(x) : 0., own ? fabs(a.b[row]) : 0., own ? fabs(r) : 0.};
-#pragma unroll
-  for(int k = 0; k < 3; ++k) {
-#pragma unroll
-    for(int o = 32; o > 0; o >>= 1) mx[k] = fmax(mx[k], __shfl_xor(mx[k], o, 64));
-    if((t & 63) == 0) psum[k][t >> 6] = mx[k];
-  }
-  resBarrier();
-  if(t < 3) {
-    double mm = 0.;
-    for(int k = 0; k < TB / 64; ++k) mm = fmax(mm, psum[t][k]);
-    a.maxima[3 * wg + t] = mm;
+  resMaxima<TB>(own, x, own ? a.b[row] : 0., r, psum, a.maxima + 3 * wg);
+}
+
+// Split-preconditioned PCG, M^-1 = G^T D^-1 G with FP32 factor values (IC(0)
+// or the learned factor), as a resident kernel: the pipelined recurrences of
+// fe_krylov.hip's spIter.  The factor has the pattern of the matrix, so it
+// adds one FP32 value per entry to the registers and no positions: G takes
+// the entries up to the diagonal, G^T those from it.  An iteration is three
+// exchanges, each with the slots of its own kind,
+//   w with the three sums:  t = D^-1 G w      (columns below the own rows)
+//   t:                      m = G^T t         (columns above)
+//   m:                      n = A m, then the vector updates,
+// where the launch-per-iteration form has three kernels that read the entries
+// again.
+// Solve with the factor's set-up, launches -> here: learned factor, P1
+// tetrahedra 30^3 (n = 24,389) 2.46 -> 0.96 ms, 45^3 (85,184) 4.40 -> 1.73, 64^3
+// (250,047, 1024 threads, part of the entries spilled) 8.70 -> 4.88; IC(0), P1
+// triangles 160^2 6.26 -> 3.25, P2 60^2 8.45 -> 4.00.  An iteration is bound by
+// its three trips of a stored word to another workgroup's poll.
+//
+// Slots come in three sets: after the sums of round k every workgroup has left
+// round k - 1, whose slots are emptied then and polled again in round k + 2;
+// the resets are complete before the sums of round k + 1 are published.
+struct SplitArgs {
+  ResArgs r;
+  const int *pos;          // per workgroup E x TB: 2 k (G) or 2 k + 1 (G^T) of each entry, -1: none
+  const float *gL, *gU, *dinv;
+};
+
+constexpr int kSplitSets = 3;
+
+// Positions of a row's entries in the factor's two CSR forms; flag: entries of
+// the factor outside the matrix's pattern.
+__global__ void splitPattern(int n, int RW, int E, int TB, const int *__restrict__ ia, const int *__restrict__ ja,
+                             const int *__restrict__ iaL, const int *__restrict__ jaL, const int *__restrict__ iaU,
+                             const int *__restrict__ jaU, int *__restrict__ pos, int *flag)
+{
+  const int wg = blockIdx.x;
+  for(int t = threadIdx.x; t < TB; t += blockDim.x) {
+    const int row = wg * RW + t;
+    const bool own = t < RW && row < n;
+    const int kb = own ? ia[row] : 0, len = own ? ia[row + 1] - kb : 0;
+    int nl = 0, nu = 0;
+    for(int e = 0; e < E; ++e) {
+      int f = -1;
+      if(e < len) {
+        const int j = ja[kb + e];
+        const int *fa = j <= row ? iaL : iaU, *fj = j <= row ? jaL : jaU;
+        for(int k = fa[row]; k < fa[row + 1] && f < 0; ++k)
+          if(fj[k] == j) f = 2 * k + (j > row);
+        if(f >= 0) j <= row ? ++nl : ++nu;
+      }
+      pos[((size_t)wg * E + e) * TB + t] = f;
+    }
+    if(own && (nl != iaL[row + 1] - iaL[row] || nu + 1 != iaU[row + 1] - iaU[row])) atomicMax(flag, 1);
   }
 }
 
 template <int TB, int E>
-int launchRes(fe_hip_ctx *ctx, FeResident &R, const ResArgs &a, size_t lds, bool *fits)
+__global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
 {
-  const void *f = (const void *)resJacobi<TB, E>;
+  const ResArgs &a = sa.r;
+  constexpr int kHeld = TB == 512 ? 3 : 2;
+  extern __shared__ double lds[];           // two regions of own + gathered values
+  __shared__ double wsum[3][4], psum[3][TB / 64];
+  __shared__ int gaveUp, below;
+  const int wg = blockIdx.x, t = threadIdx.x, G = a.G, RW = a.RW, stride = RW + a.H;
+  const int r0 = wg * RW, row = r0 + t;
+  const bool own = t < RW && row < a.n;
+  const int oT = a.n, oM = 2 * a.n, oS = 3 * a.n;
+  const size_t bufLen = 3 * ((size_t)a.n + G);
+  const int hc = a.hcnt[wg];
+  const int *hcol = a.hcol + (size_t)wg * a.hcap;
+  if(t == 0) {
+    gaveUp = 0;
+    below = 0;
+  }
+  for(int q = t; q < 2 * stride; q += TB) lds[q] = 0.;  // a factor reads only the columns of its half
+  __syncthreads();
+  for(int h = t; h < hc; h += TB)
+    if(hcol[h] < r0) atomicAdd(&below, 1);
+  double v[E];
+  float g[E], dinv = 0.f;
+  unsigned ix[E / 2], low = 0, up = 0;  // bits: entries up to, from the diagonal
+  double x = 0., r = 0., u = 0., w = 0., z = 0., q = 0., s = 0., p = 0., m = 0.;
+#pragma unroll
+  for(int e = 0; e < E / 2; ++e) ix[e] = a.idx[((size_t)wg * (E / 2) + e) * TB + t];
+  {
+    int kb = 0, len = 0;
+    if(own) {
+      kb = a.ia[row];
+      len = a.ia[row + 1] - kb;
+      r = a.b[row];
+      dinv = sa.dinv[row];
+    }
+#pragma unroll
+    for(int e = 0; e < E; ++e) {
+      const int f = sa.pos[((size_t)wg * E + e) * TB + t];
+      v[e] = e < len ? a.val[kb + e] : 0.;
+      g[e] = f < 0 ? 0.f : f & 1 ? sa.gU[f >> 1] : sa.gL[f >> 1];
+      if(e < len) {
+        const int j = a.ja[kb + e];
+        if(j <= row) low |= 1u << e;
+        if(j >= row) up |= 1u << e;
+      }
+    }
+  }
+  int hcl[kHeld];
+#pragma unroll
+  for(int k = 0; k < kHeld; ++k) hcl[k] = t + k * TB < hc ? hcol[t + k * TB] : -1;
+  resBarrier();
+  const int hLow = below;  // hcol increases: these come first
+  unsigned long long *buf = a.buf;
+  int turn = 0;
+  double *reg = lds;
+  // Own value into the slots o + row and the region, the others' gathered rows
+  // [h0, h1) from theirs; with kSum three partial sums, folded into f.
+  auto exchange = [&](auto withSums, int o, double own1, int h0, int h1, const double (&sum)[3], double (&f)[3]) -> bool {
+    constexpr bool kSum = decltype(withSums)::value;
+    reg = lds + turn * stride;
+    turn ^= 1;
+    if(own) resStore(buf + o + row, own1);
+    if(t < RW) reg[t] = own1;
+    if constexpr(kSum) {
+#pragma unroll
+      for(int j = 0; j < 3; ++j) {
+        const double ws = resWaveSum(own ? sum[j] : 0.);
+        if((t & 63) == 0) psum[j][t >> 6] = ws;
+      }
+      resBarrier();
+      if(t < 3) {
+        double ws = 0.;
+#pragma unroll
+        for(int k = 0; k < TB / 64; ++k) ws += psum[t][k];
+        resStore(buf + oS + t * G + wg, ws);
+      }
+    }
+    constexpr int kS = kSum ? 3 : 0;
+    unsigned long long pv[kS + kHeld];
+    int at[kS + kHeld];
+    if constexpr(kSum) {
+#pragma unroll
+      for(int j = 0; j < 3; ++j) at[j] = t < G ? oS + j * G + t : -1;
+    }
+#pragma unroll
+    for(int k = 0; k < kHeld; ++k) {
+      const int h = t + k * TB;
+      at[kS + k] = h >= h0 && h < h1 ? o + hcl[k] : -1;
+    }
+    bool ok = resPoll<kS + kHeld>(buf, at, pv);
+#pragma unroll
+    for(int k = 0; k < kHeld; ++k)
+      if(at[kS + k] >= 0) reg[RW + t + k * TB] = __longlong_as_double((long long)pv[kS + k]);
+    for(int h = t + kHeld * TB; h < h1 && ok; h += TB) {
+      if(h < h0) continue;
+      const int a1[1] = {o + hcol[h]};
+      unsigned long long v1[1];
+      ok = resPoll<1>(buf, a1, v1);
+      reg[RW + h] = __longlong_as_double((long long)v1[0]);
+    }
+    if(!ok) gaveUp = 1;
+    if constexpr(kSum) {
+      if(t < ((G + 63) & ~63)) {
+#pragma unroll
+        for(int j = 0; j < 3; ++j) {
+          const double ws = resWaveSum(t < G ? __longlong_as_double((long long)pv[j]) : 0.);
+          if((t & 63) == 0) wsum[j][t >> 6] = ws;
+        }
+      }
+    }
+    resBarrier();
+    if(gaveUp) return false;
+    if constexpr(kSum) {
+#pragma unroll
+      for(int j = 0; j < 3; ++j) {
+        double ws = 0.;
+        for(int k = 0; k < (G + 63) / 64; ++k) ws += wsum[j][k];
+        f[j] = resUniform(ws);
+      }
+    }
+    return true;
+  };
+  auto product = [&]() {  // the matrix
+    double y = 0.;
+#pragma unroll
+    for(int e = 0; e < E / 2; ++e) {
+      asm volatile("" : "+v"(ix[e]));  // unpacked here, not kept unpacked across the loop
+      y += v[2 * e] * reg[ix[e] & 0xffffu];
+      y += v[2 * e + 1] * reg[ix[e] >> 16];
+      if constexpr(TB == 1024 || E == 24)
+        if(e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+v"(y));
+    return y;
+  };
+  auto factor = [&](unsigned half) {  // G or G^T: the entries with their bit set
+    double y = 0.;
+    asm volatile("" : "+v"(half));
+#pragma unroll
+    for(int e = 0; e < E / 2; ++e) {
+      asm volatile("" : "+v"(ix[e]), "+v"(g[2 * e]), "+v"(g[2 * e + 1]));  // nor converted
+      const float g0 = half & (1u << (2 * e)) ? g[2 * e] : 0.f, g1 = half & (2u << (2 * e)) ? g[2 * e + 1] : 0.f;
+      y += (double)g0 * reg[ix[e] & 0xffffu];
+      y += (double)g1 * reg[ix[e] >> 16];
+      if constexpr(TB == 1024 || E == 24)
+        if(e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // eight reads in flight, not a register for each
+    }
+    asm volatile("" : "+v"(y));  // summed here, not where it is used
+    return y;
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  // uniform state (every workgroup folds the same sums in the same order)
+  double alphaP = __builtin_inf(), gammaP = 1., bn = 0., rn = 0., target = 0., tol2 = 0.;
+  int code = 0, it = 0, outer = 0, breakdowns = 0, reason = 0;
+  bool start = true;
+  for(int k = 0;; ++k) {
+    buf = a.buf + (k % kSplitSets) * bufLen;
+    double sum[3] = {r * r, 0., 0.}, f[3];
+    if(!start) {
+      sum[0] = r * u;
+      sum[1] = w * u;
+      sum[2] = r * r;
+    }
+    resStoresDone();  // the resets of the previous round
+    if(!exchange(Yes{}, 0, start ? r : w, 0, hLow, sum, f)) break;
+    {  // the slots of round k + 2 are empty again
+      unsigned long long *rs = a.buf + ((k + 2) % kSplitSets) * bufLen;
+      if(own) {
+        resStore(rs + row, kSentinel);
+        resStore(rs + oT + row, kSentinel);
+        resStore(rs + oM + row, kSentinel);
+      }
+      if(t < 3) resStore(rs + oS + t * G + wg, kSentinel);
+    }
+    double alpha = 0., beta = 0.;
+    if(start) {
+      rn = resUniform(sqrt(f[0]));  // ||b||, or the true residual's norm
+      if(outer == 0) {
+        bn = rn;
+        target = resUniform(fmax(a.rtol * bn, a.atol));
+        tol2 = resUniform(target * target * 0.25);
+        if(bn == 0.) reason = 2;
+      } else {
+        if(rn <= target) reason = 2;
+        else if(code == 4 || !(rn == rn)) reason = -9;
+        else if(it >= a.maxit) reason = -3;
+        else if(rn / bn > a.dtol) reason = -4;
+        else if(code == 3 && ++breakdowns > 20) reason = -3;
+        code = 0;  // again from the true residual
+      }
+      if(reason) break;
+      z = q = s = p = 0.;
+      gammaP = 1.;
+      alphaP = __builtin_inf();
+    } else {
+      if(!(f[2] > tol2) || it >= a.maxit) {
+        code = f[2] <= tol2 ? 1 : (f[2] == f[2] ? 2 : 4);
+      } else {
+        beta = resUniform(f[0] / gammaP);
+        const double den = f[1] - beta * f[0] / alphaP;
+        if(den > 0.) {
+          alpha = resUniform(f[0] / den);
+          gammaP = f[0];
+          alphaP = alpha;
+          ++it;
+        } else {
+          code = 3;  // breakdown: the preconditioned operator is not SPD
+        }
+      }
+      if(code) {  // the true residual
+        if(!exchange(No{}, oM, x, 0, hc, sum, f)) break;
+        r = own ? a.b[row] - product() : 0.;
+        ++outer;
+        start = true;
+        continue;
+      }
+    }
+    const double tv = (double)dinv * factor(low);
+    if(!exchange(No{}, oT, tv, hLow, hc, sum, f)) break;
+    m = factor(up);
+    if(!exchange(No{}, oM, m, 0, hc, sum, f)) break;
+    const double y = product();
+    if(start) {
+      u = m;
+      w = y;
+      start = false;
+    } else {
+      z = y + beta * z;
+      q = m + beta * q;
+      s = w + beta * s;
+      p = u + beta * p;
+      x = x + alpha * p;
+      r = r - alpha * s;
+      u = u - alpha * q;
+      w = w - alpha * z;
+    }
+  }
+  if(t == 0) {
+    if(gaveUp) __hip_atomic_store(&a.out->gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if(wg == 0) {
+      a.out->reason = reason;
+      a.out->iters = it;
+      a.out->outer = outer;
+      a.out->bn = bn;
+      a.out->rn = rn;
+    }
+  }
+  if(own) a.x[row] = x;
+  resMaxima<TB>(own, x, own ? a.b[row] : 0., r, psum, a.maxima + 3 * wg);
+}
+
+template <typename Args>
+int launchRes(fe_hip_ctx *ctx, void (*kernel)(Args), int TB, const FeResident &R, const Args &a, size_t lds, bool *fits)
+{
+  const void *f = (const void *)kernel;
   int perCu = 0, cus = 0;
   *fits = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, f, TB, lds) == hipSuccess &&
@@ -407,17 +728,9 @@ int launchRes(fe_hip_ctx *ctx, FeResident &R, const ResArgs &a, size_t lds, bool
     (void)hipGetLastError();
     return FE_STATUS_OK;
   }
-  hipLaunchKernelGGL((resJacobi<TB, E>), dim3(R.G), dim3(TB), lds, ctx->stream, a);
+  hipLaunchKernelGGL(kernel, dim3(R.G), dim3(TB), lds, ctx->stream, a);
   FE_HIP_TRY(ctx, hipGetLastError());
   return FE_STATUS_OK;
-}
-
-template <int TB>
-int launchResE(fe_hip_ctx *ctx, FeResident &R, const ResArgs &a, size_t lds, bool *fits)
-{
-  if(R.E == 8) return launchRes<TB, 8>(ctx, R, a, lds, fits);
-  if(R.E == 16) return launchRes<TB, 16>(ctx, R, a, lds, fits);
-  return launchRes<TB, 24>(ctx, R, a, lds, fits);
 }
 
 int resBuild(fe_hip_ctx *ctx, FeResident &R)
@@ -469,31 +782,21 @@ std::mutex &feResidentMutex(int device)
   return m[device & 63];
 }
 
-int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res)
+namespace {
+
+// One resident launch over `bufLen` slots, and what it returned.  launch(&fits)
+// enqueues the kernel.
+template <typename F>
+int resRun(fe_hip_ctx *ctx, FeResident &R, unsigned long long *buf, size_t cells, FeResidentResult *res, F launch)
 {
-  res->ran = false;
-  if(!ctx->resident || ctx->residentGaveUp) return FE_STATUS_OK;
-  if(!ctx->res) ctx->res = new FeResident();
-  FeResident &R = *ctx->res;
-  if(!R.built)
-    if(int rc = resBuild(ctx, R)) return rc;
-  if(!R.usable) return FE_STATUS_OK;
-  const int hcap = std::min(kResH, kResLds / 16 - R.RW);
-  const ResArgs a{ctx->n,     R.G,     R.RW, R.H,     hcap,    ctx->d_ia, ctx->d_ja,       ctx->d_val, R.d_idx, R.d_hcol,
-                  R.d_hcnt,   ctx->d_rhs, x, R.d_buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter};
-  const size_t lds = 2 * (size_t)(R.RW + R.H) * sizeof(double);
-  const size_t cells = kResBufs * ((size_t)ctx->n + 3 * (size_t)R.G);
   bool fits = false;
   {
     std::lock_guard<std::mutex> lock(feResidentMutex(ctx->device));
     if(ctx->profiling)
       if(int rc = feTimerMark(ctx, ctx->spmvTimer)) return rc;
     hipLaunchKernelGGL(resFill, dim3((unsigned)std::min<size_t>(1024, (cells + 255) / 256)), dim3(256), 0, ctx->stream,
-                       cells, R.d_buf, R.d_out);
-    int rc = FE_STATUS_OK;
-    if(R.TB == 512) rc = launchResE<512>(ctx, R, a, lds, &fits);
-    else rc = launchResE<1024>(ctx, R, a, lds, &fits);
-    if(rc) return rc;
+                       cells, buf, R.d_out);
+    if(int rc = launch(&fits)) return rc;
     if(fits) {
       if(ctx->profiling)
         if(int rc2 = feTimerMark(ctx, ctx->spmvTimer)) return rc2;
@@ -530,6 +833,72 @@ int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, Fe
     t.used = 0;
   }
   return FE_STATUS_OK;
+}
+
+int resPrepare(fe_hip_ctx *ctx)
+{
+  if(!ctx->res) ctx->res = new FeResident();
+  if(!ctx->res->built) return resBuild(ctx, *ctx->res);
+  return FE_STATUS_OK;
+}
+
+ResArgs resArgs(const fe_hip_ctx *ctx, const FeResident &R, const fe_hip_solver_opts *o, double *x,
+                unsigned long long *buf)
+{
+  const int hcap = std::min(kResH, kResLds / 16 - R.RW);
+  return ResArgs{ctx->n,   R.G,        R.RW, R.H, hcap,    ctx->d_ia, ctx->d_ja,       ctx->d_val, R.d_idx, R.d_hcol,
+                 R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter};
+}
+
+}  // namespace
+
+int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res)
+{
+  res->ran = false;
+  if(!ctx->resident || ctx->residentGaveUp) return FE_STATUS_OK;
+  if(int rc = resPrepare(ctx)) return rc;
+  FeResident &R = *ctx->res;
+  if(!R.usable) return FE_STATUS_OK;
+  const ResArgs a = resArgs(ctx, R, o, x, R.d_buf);
+  const size_t lds = 2 * (size_t)(R.RW + R.H) * sizeof(double);
+  return resRun(ctx, R, R.d_buf, kResBufs * ((size_t)ctx->n + 3 * (size_t)R.G), res, [&](bool *fits) {
+    auto *const k = R.TB == 512 ? (R.E == 8 ? resJacobi<512, 8> : R.E == 16 ? resJacobi<512, 16> : resJacobi<512, 24>)
+                                : (R.E == 8 ? resJacobi<1024, 8> : R.E == 16 ? resJacobi<1024, 16> : resJacobi<1024, 24>);
+    return launchRes(ctx, k, R.TB, R, a, lds, fits);
+  });
+}
+
+int feResidentSplit(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeResidentResult *res)
+{
+  res->ran = false;
+  if(!ctx->resident || ctx->residentGaveUp || !ctx->pcValues32 || ctx->pcFp32) return FE_STATUS_OK;
+  if(int rc = resPrepare(ctx)) return rc;
+  FeResident &R = *ctx->res;
+  // 1024 threads have no registers for longer rows
+  if(!R.usable || R.splitState < 0 || (R.TB == 1024 && R.E > 16)) return FE_STATUS_OK;
+  const FePrecond &P = ctx->pc;
+  const size_t cells = kSplitSets * 3 * ((size_t)ctx->n + R.G);
+  if(R.splitState == 0) {
+    int *flag = nullptr, bad = 0;
+    if(feAlloc(ctx, &flag, 1) || feAlloc(ctx, &R.d_pos, (size_t)R.G * R.E * R.TB) || feAlloc(ctx, &R.d_splitBuf, cells))
+      return FE_STATUS_OUT_OF_MEMORY;
+    FE_HIP_TRY(ctx, hipMemsetAsync(flag, 0, sizeof(int), ctx->stream));
+    hipLaunchKernelGGL(splitPattern, dim3(R.G), dim3(512), 0, ctx->stream, ctx->n, R.RW, R.E, R.TB, ctx->d_ia, ctx->d_ja,
+                       P.d_iaL, P.d_jaL, P.d_iaU, P.d_jaU, R.d_pos, flag);
+    FE_HIP_TRY(ctx, hipGetLastError());
+    FE_HIP_TRY(ctx, hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    feFree(ctx, flag);
+    R.splitState = bad ? -1 : 1;
+    if(bad) return FE_STATUS_OK;
+  }
+  const SplitArgs a{resArgs(ctx, R, o, x, R.d_splitBuf), R.d_pos, P.d_gL32, P.d_gU32, P.d_dinv32};
+  const size_t lds = 2 * (size_t)(R.RW + R.H) * sizeof(double);
+  return resRun(ctx, R, R.d_splitBuf, cells, res, [&](bool *fits) {
+    auto *const k = R.TB == 512 ? (R.E == 8 ? resSplit<512, 8> : R.E == 16 ? resSplit<512, 16> : resSplit<512, 24>)
+                                : (R.E == 8 ? resSplit<1024, 8> : resSplit<1024, 16>);
+    return launchRes(ctx, k, R.TB, R, a, lds, fits);
+  });
 }
 
 void feResidentRelease(fe_hip_ctx *ctx)

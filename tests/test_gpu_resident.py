@@ -83,3 +83,47 @@ def test_resident_two_threads():
         assert np.array_equal(g, w)
     for S in systems:
         S.close()
+
+
+# rows of 8, 16 and 24 entries; one workgroup, its edge, many; 1024 threads (4, 52); rows too long (5, 6)
+@pytest.mark.parametrize("pc", ["ic0", "learned"])
+@pytest.mark.parametrize("kind, N", [(1, 2), (1, 3), (1, 24), (1, 150), (4, 3), (4, 9), (4, 30), (4, 52), (2, 12), (2, 90),
+                                     (5, 6)])
+def test_resident_split_equals_launch_per_iteration(kind, N, pc):
+    from feng_amd.api import PC_IC0, PC_LEARNED
+    print("resident split", kind, N, pc, flush=True)
+    S, num = _system(kind, N)
+    if pc == "learned":
+        from feng_amd.learned import load_weights
+        load_weights(S)
+    pcn = PC_IC0 if pc == "ic0" else PC_LEARNED
+    out = {}
+    for resident in (0, 1):
+        S.set_tuning("resident", resident)
+        out[resident] = S.solve(pc=pcn, rtol=1e-9, max_iter=20000, want_du=True)
+    (r0, x0), (r1, x1) = out[0], out[1]
+    if not r0.converged:  # a learned factor outside its training range: no iteration is possible in either form
+        assert r0.iterations == r1.iterations == 0 and r1.reason == r0.reason
+        S.close()
+        return
+    assert r1.converged and r1.relres <= 1e-9
+    # as above: the same recurrences with sums in another order
+    if r0.outer_iterations == r1.outer_iterations == 1:
+        assert abs(r1.iterations - r0.iterations) <= 2 + r0.iterations // 20
+    assert np.linalg.norm(x1 - x0) <= 1e-6 * np.linalg.norm(x0)
+    ia, ja = S.get_csr()
+    val, rhs = S.get_system()
+    res = rhs - np.add.reduceat(val * x1[ja], ia[:-1])
+    assert np.linalg.norm(res) <= 1.02e-9 * np.linalg.norm(rhs)
+    assert r1.norm_rhs_inf == np.abs(rhs).max() and r1.norm_dx_inf == np.abs(x1).max()
+    again, x2 = S.solve(pc=pcn, rtol=1e-9, max_iter=20000, want_du=True)
+    assert again.iterations == r1.iterations and np.array_equal(x1, x2)  # bitwise repeatable
+    if r1.iterations > 6:
+        rb, xb = S.solve(pc=pcn, rtol=1e-9, max_iter=5, want_du=True)
+        assert not rb.converged and rb.reason == -3 and rb.iterations == 5
+        rr = np.linalg.norm(rhs - np.add.reduceat(val * xb[ja], ia[:-1])) / np.linalg.norm(rhs)
+        assert abs(rb.relres - rr) <= 1e-9 * rr
+    S.set_system(rhs=np.zeros_like(rhs))
+    rz, xz = S.solve(pc=pcn, want_du=True)
+    assert rz.converged and rz.iterations == 0 and not xz.any()
+    S.close()

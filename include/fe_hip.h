@@ -99,7 +99,10 @@ typedef struct {
 #define FE_PC_FIELDSPLIT 7
 
 #define FE_PREC_FP64 0    /* FP64 Krylov */
-#define FE_PREC_FP32_IR 1 /* FP32 inner Krylov + FP64 iterative refinement (multigrid-PCG: FP64 up to 700,000 rows) */
+/* FP32 inner Krylov + FP64 iterative refinement; CG runs in FP64 instead where
+ * that is faster: solves that fit one launch (about 260,000 rows of at most 24
+ * entries), multigrid-PCG up to 700,000 rows */
+#define FE_PREC_FP32_IR 1
 
 typedef struct {
   int ksp;           /* FE_KSP_* */

@@ -114,6 +114,7 @@ struct ArArgs {
   double *maxima;
   double rtol, atol, dtol, oc;
   int maxit;
+  long long wait;  // ticks
 };
 
 // LDS positions of the columns of a workgroup's rows (see fe_resident.hip):
@@ -467,14 +468,14 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
     }
 #pragma unroll
     for(int k = 0; k < kHeld; ++k) at[kS + k] = hcl[k] >= 0 ? o + hcl[k] : -1;
-    bool ok = resPoll<kS + kHeld>(buf, at, pv);
+    bool ok = resPoll<kS + kHeld>(buf, at, pv, a.wait);
 #pragma unroll
     for(int k = 0; k < kHeld; ++k)
       if(hcl[k] >= 0) reg[L0.rows + t + k * kTB] = __longlong_as_double((long long)pv[kS + k]);
     for(int h = t + kHeld * kTB; h < hc0 && ok; h += kTB) {
       const int a1[1] = {o + hcol0[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1);
+      ok = resPoll<1>(buf, a1, v1, a.wait);
       reg[L0.rows + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;
@@ -553,7 +554,7 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
     for(int h = t; h < hc && ok; h += kTB) {
       const int a1[1] = {o + hcol[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1);
+      ok = resPoll<1>(buf, a1, v1, a.wait);
       reg[L.rows + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;
@@ -721,7 +722,7 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
       for(int i = t; i < a.parts && ok; i += 2 * kTB) {
         const int a2[2] = {a.oParts + i, i + kTB < a.parts ? a.oParts + i + kTB : -1};
         unsigned long long v2[2];
-        ok = resPoll<2>(buf, a2, v2);
+        ok = resPoll<2>(buf, a2, v2, a.wait);
         parts[i] = __longlong_as_double((long long)v2[0]);
         if(i + kTB < a.parts) parts[i + kTB] = __longlong_as_double((long long)v2[1]);
       }
@@ -1135,6 +1136,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
   a.dtol = o->dtol;
   a.oc = ctx->amgOverCorrect;
   a.maxit = o->max_iter;
+  a.wait = resWaitTicks(ctx);
   bool fits = false;
   {
     std::lock_guard<std::mutex> lock(feResidentMutex(ctx->device));
@@ -1174,7 +1176,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
     return FE_STATUS_OK;
   }
   FE_REQUIRE(ctx, out.bn == 0. || !out.badPivot, "AMG: the coarsest operator is not positive definite");
-  res->ran = true;
+  res->ran = ctx->residentRan = true;
   res->reason = out.reason;
   res->iters = out.iters;
   res->outer = out.outer;

@@ -754,6 +754,10 @@ int fe_hip_set_tuning(fe_hip_ctx *ctx, const char *key, int value)
   } else if(k == "resident") {
     FE_REQUIRE(ctx, value == 0 || value == 1, "resident must be 0 or 1");
     ctx->resident = value;
+    ctx->residentGaveUp = false;
+  } else if(k == "resident_wait_us") {
+    FE_REQUIRE(ctx, value >= 0 && value <= 1000000, "resident_wait_us must be in [0, 1000000]");
+    ctx->residentWaitUs = value;
   } else if(k == "ilu_sweeps") {
     FE_REQUIRE(ctx, value >= 0 && value <= 64,
                "ilu_sweeps must be 0 (exact triangular solves) or a sweep count in [1, 64]");
@@ -849,6 +853,9 @@ int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value)
   else if(k == "ic0_sweeps") *value = ctx->icSweeps;
   else if(k == "ilu_sweeps") *value = ctx->pc.sweeps;
   else if(k == "resident") *value = ctx->resident;
+  else if(k == "resident_wait_us") *value = ctx->residentWaitUs;
+  else if(k == "resident_ran") *value = ctx->residentRan;
+  else if(k == "resident_gave_up") *value = ctx->residentGaveUp;
   else if(k == "gmres_orth") *value = ctx->gmresOrth;
   else if(k == "pc_fp32") *value = ctx->pcFp32;
   else if(k == "pc_values32") *value = ctx->pcValues32;

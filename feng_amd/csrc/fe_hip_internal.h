@@ -205,8 +205,10 @@ struct fe_hip_ctx {
   FeTriSolve *tri = nullptr;
   FeResident *res = nullptr;
   FeAmgResident *amgRes = nullptr;
-  int resident = 1;             // FP64 Jacobi- and multigrid-PCG: all iterations in one launch where the system fits (0: never)
-  bool residentGaveUp = false;  // a wait of a resident launch ran out: this context keeps the other kernels
+  int resident = 1;             // CG: all iterations in one launch where the system fits (0: never)
+  int residentWaitUs = 50000;   // longest wait of such a launch for another workgroup's value
+  bool residentRan = false;     // the last solve was one
+  bool residentGaveUp = false;  // a wait ran out: the other kernels until the tuning key `resident` is set again
 
   // mesh
   int dim = 0, V = 0, E = 0, nvpe = 0;

@@ -1704,6 +1704,7 @@ int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out)
 int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip_solve_stats *stats)
 {
   const fe_hip_solver_opts *o = given;
+  ctx->residentRan = false;
   if(o->ksp == FE_KSP_GMRES) return feSolveGmres(ctx, o, du, stats);
   if(o->ksp == FE_KSP_DIRECT) return feSolveDirect(ctx, o, du, stats);
   FE_REQUIRE(ctx, o->ksp == FE_KSP_CG, "unknown Krylov method");

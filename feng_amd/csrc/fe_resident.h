@@ -15,9 +15,10 @@
 // and the reset is complete (vmcnt 0) before the owner publishes its part of
 // exchange q + 1, which any workgroup receives before it polls exchange q + 2.
 //
-// Every wait is bounded by wall time (kResWaitTicks): a workgroup that gives
-// up raises a flag and leaves, later waits of the launch give up the same
-// way, and the host repeats the solve with the launch-per-iteration kernels.
+// Every wait is bounded by wall time (50 ms, tuning key resident_wait_us): a
+// workgroup that gives up raises a flag and leaves, later waits of the launch
+// give up the same way, and the host repeats the solve with the
+// launch-per-iteration kernels.
 // All workgroups of a launch must be resident together: the host checks the
 // occupancy and lets one resident launch run per device at a time.
 #pragma once
@@ -32,7 +33,6 @@ std::mutex &feResidentMutex(int device);
 namespace fe_res {
 
 constexpr unsigned long long kSentinel = 0x7FF4DEAD5EA7F00Dull;
-constexpr long long kResWaitTicks = 5000000;  // 50 ms of the 100 MHz counter
 constexpr int kResBufs = 4;
 
 __device__ __forceinline__ unsigned long long resLoad(const unsigned long long *p)
@@ -50,10 +50,18 @@ __device__ __forceinline__ void resBarrier() { asm volatile("s_waitcnt lgkmcnt(0
 // Every global store of this wavefront has reached its coherence point.
 __device__ __forceinline__ void resStoresDone() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// The longest wait of a launch, in ticks of the 100 MHz counter; 0 us: no wait
+// at all, give up on the first value that has not arrived.
+inline long long resWaitTicks(const fe_hip_ctx *ctx)
+{
+  return ctx->residentWaitUs > 0 ? 100ll * ctx->residentWaitUs : -1;
+}
+
 // Polls the K slots base[idx[k]] (idx < 0: none) until all have arrived; false
 // when the time is up.  The loads of a round are issued together.
 template <int K>
-__device__ __forceinline__ bool resPoll(const unsigned long long *base, const int (&idx)[K], unsigned long long (&v)[K])
+__device__ __forceinline__ bool resPoll(const unsigned long long *base, const int (&idx)[K], unsigned long long (&v)[K],
+                                        long long ticks)
 {
 #pragma unroll
   for(int k = 0; k < K; ++k) v[k] = idx[k] >= 0 ? resLoad(base + (unsigned)idx[k]) : 0ull;
@@ -71,7 +79,7 @@ __device__ __forceinline__ bool resPoll(const unsigned long long *base, const in
         all = all && v[k] != kSentinel;
       }
     if(all) return true;
-    if(wall_clock64() - t0 > kResWaitTicks) return false;
+    if(wall_clock64() - t0 > ticks) return false;
   }
 }
 

@@ -75,6 +75,7 @@ struct ResArgs {
   double *maxima;
   double rtol, atol, dtol;
   int maxit;
+  long long wait;  // ticks
 };
 
 // LDS positions of a workgroup's entries: own rows first, then the other
@@ -267,14 +268,14 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
 #pragma unroll
       for(int k = 0; k < 3; ++k)
         if(!kSplit || t < sumThreads) at[k] = t < G ? a.n + k * G + t : -1;
-      bool ok = resPoll<kPoll>(buf, at, pv);
+      bool ok = resPoll<kPoll>(buf, at, pv, a.wait);
 #pragma unroll
       for(int k = 0; k < kHeld; ++k)
         if(hcl[k] >= 0) reg[RW + h0 + k * hStep] = __longlong_as_double((long long)pv[kSums + k]);
       for(int h = h0 + kHeld * hStep; h0 >= 0 && h < hc && ok; h += hStep) {
         const int a1[1] = {hcol[h]};
         unsigned long long v1[1];
-        ok = resPoll<1>(buf, a1, v1);
+        ok = resPoll<1>(buf, a1, v1, a.wait);
         reg[RW + h] = __longlong_as_double((long long)v1[0]);
       }
       if(t < G) {
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
       const int h = t + k * TB;
       at[kS + k] = h >= h0 && h < h1 ? o + hcl[k] : -1;
     }
-    bool ok = resPoll<kS + kHeld>(buf, at, pv);
+    bool ok = resPoll<kS + kHeld>(buf, at, pv, a.wait);
 #pragma unroll
     for(int k = 0; k < kHeld; ++k)
       if(at[kS + k] >= 0) reg[RW + t + k * TB] = __longlong_as_double((long long)pv[kS + k]);
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
       if(h < h0) continue;
       const int a1[1] = {o + hcol[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1);
+      ok = resPoll<1>(buf, a1, v1, a.wait);
       reg[RW + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;
@@ -816,7 +817,7 @@ int resRun(fe_hip_ctx *ctx, FeResident &R, unsigned long long *buf, size_t cells
     ctx->residentGaveUp = true;
     return FE_STATUS_OK;
   }
-  res->ran = true;
+  res->ran = ctx->residentRan = true;
   res->reason = out.reason;
   res->iters = out.iters;
   res->outer = out.outer;
@@ -847,7 +848,8 @@ ResArgs resArgs(const fe_hip_ctx *ctx, const FeResident &R, const fe_hip_solver_
 {
   const int hcap = std::min(kResH, kResLds / 16 - R.RW);
   return ResArgs{ctx->n,   R.G,        R.RW, R.H, hcap,    ctx->d_ia, ctx->d_ja,       ctx->d_val, R.d_idx, R.d_hcol,
-                 R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter};
+                 R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter,
+                 resWaitTicks(ctx)};
 }
 
 }  // namespace

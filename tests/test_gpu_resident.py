@@ -31,6 +31,9 @@ def test_resident_equals_launch_per_iteration(kind, N):
     for resident in (0, 1):
         S.set_tuning("resident", resident)
         out[resident] = S.solve(rtol=1e-9, max_iter=20000, want_du=True)
+        # more than one row a thread of the device, or rows of more than 24 entries, do not fit
+        fits = S.n <= 262144 and kind != 5
+        assert S.get_tuning("resident_ran") == (resident and fits) and S.get_tuning("resident_gave_up") == 0
     (r0, x0), (r1, x1) = out[0], out[1]
     assert r0.converged and r1.converged and r1.relres <= 1e-9
     # the same recurrences with sums in another order: the stop moves by a few
@@ -82,7 +85,35 @@ def test_resident_two_threads():
     for g, w in zip(got, want):
         assert np.array_equal(g, w)
     for S in systems:
+        assert S.get_tuning("resident_ran") == 1 and S.get_tuning("resident_gave_up") == 0
         S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0", "amg"])
+def test_a_wait_that_runs_out_leaves_the_solve_to_the_launches(pc):
+    """No waiting at all: the first value of another workgroup that has not
+    arrived ends the launch.  The solve is the launch-per-iteration one bit for
+    bit, later solves stay there, and setting `resident` again tries anew."""
+    from feng_amd.api import PC_AMG, PC_IC0, PC_JACOBI
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0, "amg": PC_AMG}[pc]
+    S, _ = _system(4, 21)
+
+    def solve():
+        return S.solve(pc=pcn, rtol=1e-9, want_du=True)
+    S.set_tuning("resident", 0)
+    r0, x0 = solve()
+    S.set_tuning("resident", 1)
+    S.set_tuning("resident_wait_us", 0)
+    for _ in range(2):
+        r1, x1 = solve()
+        assert S.get_tuning("resident_ran") == 0 and S.get_tuning("resident_gave_up") == 1
+        assert r1.converged and r1.iterations == r0.iterations and np.array_equal(x1, x0)
+    S.set_tuning("resident_wait_us", 50000)
+    S.set_tuning("resident", 1)
+    r2, x2 = solve()
+    assert S.get_tuning("resident_ran") == 1 and S.get_tuning("resident_gave_up") == 0
+    assert r2.converged and np.linalg.norm(x2 - x0) <= 1e-6 * np.linalg.norm(x0)
+    S.close()
 
 
 # rows of 8, 16 and 24 entries; one workgroup, its edge, many; 1024 threads (4, 52); rows too long (5, 6)
@@ -101,6 +132,7 @@ def test_resident_split_equals_launch_per_iteration(kind, N, pc):
     for resident in (0, 1):
         S.set_tuning("resident", resident)
         out[resident] = S.solve(pc=pcn, rtol=1e-9, max_iter=20000, want_du=True)
+        assert S.get_tuning("resident_ran") == (resident and kind != 5) and S.get_tuning("resident_gave_up") == 0
     (r0, x0), (r1, x1) = out[0], out[1]
     if not r0.converged:  # a learned factor outside its training range: no iteration is possible in either form
         assert r0.iterations == r1.iterations == 0 and r1.reason == r0.reason

@@ -755,6 +755,9 @@ int fe_hip_set_tuning(fe_hip_ctx *ctx, const char *key, int value)
     FE_REQUIRE(ctx, value == 0 || value == 1, "resident must be 0 or 1");
     ctx->resident = value;
     ctx->residentGaveUp = false;
+  } else if(k == "amg_fp32_rows") {
+    FE_REQUIRE(ctx, value >= 0, "amg_fp32_rows must be >= 0 (0: FP32 iterations for every system)");
+    ctx->amgFp32Rows = value;
   } else if(k == "resident_wait_us") {
     FE_REQUIRE(ctx, value >= 0 && value <= 1000000, "resident_wait_us must be in [0, 1000000]");
     ctx->residentWaitUs = value;
@@ -853,6 +856,7 @@ int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value)
   else if(k == "ic0_sweeps") *value = ctx->icSweeps;
   else if(k == "ilu_sweeps") *value = ctx->pc.sweeps;
   else if(k == "resident") *value = ctx->resident;
+  else if(k == "amg_fp32_rows") *value = ctx->amgFp32Rows;
   else if(k == "resident_wait_us") *value = ctx->residentWaitUs;
   else if(k == "resident_ran") *value = ctx->residentRan;
   else if(k == "resident_gave_up") *value = ctx->residentGaveUp;
@@ -868,6 +872,7 @@ int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value)
   else if(k == "amg_pad_tiles") *value = ctx->amgPadTiles;
   else if(k == "batch_amg_global") *value = ctx->batchAmgGlobal;
   else if(k == "graph_iters") *value = ctx->graphIters;
+  else if(k == "graphs") *value = (int)ctx->graphs.size();
   else FE_REQUIRE(ctx, false, "unknown tuning key " + k);
   return FE_STATUS_OK;
 }

@@ -205,6 +205,7 @@ struct fe_hip_ctx {
   FeTriSolve *tri = nullptr;
   FeResident *res = nullptr;
   FeAmgResident *amgRes = nullptr;
+  int amgFp32Rows = 700000;     // multigrid-PCG at FE_PREC_FP32_IR: FP32 iterations above this many rows, FP64 ones up to it
   int resident = 1;             // CG: all iterations in one launch where the system fits (0: never)
   int residentWaitUs = 50000;   // longest wait of such a launch for another workgroup's value
   bool residentRan = false;     // the last solve was one

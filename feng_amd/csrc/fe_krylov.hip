@@ -1692,8 +1692,6 @@ __global__ void castResidual(int n, const double *__restrict__ a, T *__restrict_
 
 }  // namespace
 
-constexpr int kAmgFp32From = 700000;
-
 int feResidualNorm2(fe_hip_ctx *ctx, const double *x, double *r, double *out)
 {
   Workspace w;
@@ -1713,7 +1711,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   const bool split = (o->pc != FE_PC_JACOBI);
   const bool amg = (o->pc == FE_PC_AMG);
   ctx->amgActive = amg;
-  // Multigrid-PCG with FP32 inner solves (FE_PREC_FP32_IR), up to kAmgFp32From
+  // Multigrid-PCG with FP32 inner solves (FE_PREC_FP32_IR), up to amgFp32Rows
   // rows: the FP64 iteration (level values stay FP32) instead.  A launch or a
   // wait costs the same in either precision, and an FP32 product needs a
   // restart or a replaced residual each time the residual has fallen by
@@ -1721,10 +1719,16 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   // rows, 1e4 contrast 80 -> 41 ms (647 -> 259 iterations), 576,081 rows,
   // constant 32.8 -> 15.2 ms; P1 triangles, 488,601 rows 9.3 -> 8.4 ms; P1
   // tetrahedra, 421,875 rows 7.2 -> 6.8 ms, level at 704,969 rows (10.9 and
-  // 11.1 ms), above which bytes decide.  Per-level kernels: P1 tetrahedra,
-  // 493,039 rows 26.1 -> 14.8 ms; P2 triangles, 249,001 rows 68.5 -> 49.5 ms.
+  // 11.1 ms).  Per-level kernels: P1 tetrahedra, 493,039 rows 26.1 -> 14.8 ms;
+  // P2 triangles, 249,001 rows 68.5 -> 49.5 ms.  The line is where P1
+  // tetrahedra turn: at 970,299 rows FP32 takes 12.9 ms and FP64 13.2.
+  // Triangles have not turned there, nor at the sizes measured above: P2, 1e4
+  // contrast, 1,046,529 rows 130 and 74 ms, 4,190,209 rows 741 and 451 ms,
+  // constant 30.8 and 30.7, 230 and 173 ms; P1, 998,001 rows 17.3 and 15.4 ms.
+  // They keep FP32 iterations above the line all the same (the line looks at
+  // no row length); FE_PREC_FP64 or a larger amg_fp32_rows is faster for them.
   fe_hip_solver_opts wide = *given;
-  if(amg && given->precision == FE_PREC_FP32_IR && ctx->d_val32 && ctx->pcValues32 && ctx->n <= kAmgFp32From) {
+  if(amg && given->precision == FE_PREC_FP32_IR && ctx->d_val32 && ctx->pcValues32 && ctx->n <= ctx->amgFp32Rows) {
     wide.precision = FE_PREC_FP64;
     o = &wide;
   }

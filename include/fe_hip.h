@@ -266,12 +266,15 @@ int fe_hip_set_profiling(fe_hip_ctx *ctx, int on);
  * multiple of 8 up to 4096); FE_PC_AMG: "amg_omega_x100" (l1-Jacobi factor
  * times 100, default 180), "amg_oc_x100" (coarse over-correction times 100,
  * default 180), "amg_block_rows" (levels up to this many rows run in one
- * workgroup, default 1024), "resident" (1, default: CG solves of systems that
- * fit in one launch; setting it clears "resident_gave_up"),
+ * workgroup, default 1024), "amg_fp32_rows" (multigrid-PCG at FE_PREC_FP32_IR
+ * iterates in FP64 up to this many rows, default 700000), "resident" (1,
+ * default: CG solves of systems that fit in one launch; setting it clears
+ * "resident_gave_up"),
  * "resident_wait_us" (longest wait of such a launch, default 50000; when one
  * runs out the solve is repeated by launches, and later solves take them too).
  * Read-only: "resident_ran" (the last solve was one launch),
- * "resident_gave_up" (a wait has run out). */
+ * "resident_gave_up" (a wait has run out), "graphs" (captured graphs the
+ * context holds). */
 int fe_hip_set_tuning(fe_hip_ctx *ctx, const char *key, int value);
 int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value);
 

@@ -136,8 +136,10 @@ def test_numeric_setup_follows_new_values():
     S.close()
 
 
+# amg_fp32_rows 0: FP32 iterations at FE_PREC_FP32_IR, as for systems of more than 700,000 rows
+@pytest.mark.parametrize("fp32_rows", [700000, 0])
 @pytest.mark.parametrize("case", ["tet_grf_16", "p2_blocks_64"])
-def test_amg_pcg_converges(oracle, case):
+def test_amg_pcg_converges(oracle, case, fp32_rows):
     from feng_amd.api import FN_CONST, FN_ELEM, PC_AMG, PC_JACOBI, PREC_FP32_IR, Fn, Mesh
     from feng_amd.problems import diffusion_system
     print("case", case, flush=True)
@@ -149,10 +151,12 @@ def test_amg_pcg_converges(oracle, case):
         k, kind, deg = Fn(FN_ELEM, data=m.coeff_blocks(16, 1e-2, 1e2, 9)), 2, 2
     S, num = diffusion_system(m, kind, deg, k, Fn(FN_CONST, -1.0))
     S.assemble(3, PREC_FP32_IR)
+    S.set_tuning("amg_fp32_rows", fp32_rows)
     rj = S.solve(pc=PC_JACOBI, rtol=1e-8, max_iter=20000)
     ra, du = S.solve(pc=PC_AMG, rtol=1e-8, want_du=True)
     ra32 = S.solve(pc=PC_AMG, precision=PREC_FP32_IR, rtol=1e-8, inner_rtol=1e-2)
     assert rj.converged and ra.converged and ra32.converged
+    assert S.get_tuning("resident_ran") == (fp32_rows > 0) and (fp32_rows > 0 or ra32.outer_iterations >= 2)
     assert ra.iterations * 3 < rj.iterations, (ra.iterations, rj.iterations)
     ia, ja = S.get_csr()
     val, rhs = S.get_system()
@@ -161,15 +165,21 @@ def test_amg_pcg_converges(oracle, case):
     S.close()
 
 
+@pytest.mark.parametrize("resident", [1, 0])
 @pytest.mark.parametrize("pcname", ["amg", "ic0"])
-def test_graph_replay_matches_direct_launches(pcname):
+def test_graph_replay_matches_direct_launches(pcname, resident):
     """Iteration batches replayed from a captured HIP graph give the same
     iterates as direct launches, bit for bit, on every replayed solve (eager
-    solves and host synchronisations in between)."""
+    solves and host synchronisations in between).  Graphs hold the pipelined
+    split and per-level multigrid iterations: a solve in one launch (resident)
+    replays none and does not change either."""
     from feng_amd.api import PC_AMG, PC_IC0, PREC_FP32_IR
     pc = {"amg": PC_AMG, "ic0": PC_IC0}[pcname]
     m, S, num = _system("tet_grf_12")
     S.assemble(3, PREC_FP32_IR)
+    if not resident:
+        for key, v in (("resident", 0), ("amg_kernel", 1), ("amg_fp32_rows", 0), ("pipe_kernel", 1)):
+            S.set_tuning(key, v)
     for prec in (0, PREC_FP32_IR):
         S.set_tuning("graph_iters", 0)
         r0, d0 = S.solve(pc=pc, precision=prec, rtol=1e-8, want_du=True)
@@ -182,6 +192,7 @@ def test_graph_replay_matches_direct_launches(pcname):
             S.set_tuning("graph_iters", 0)
             r2, d2 = S.solve(pc=pc, precision=prec, rtol=1e-8, want_du=True)
             assert np.array_equal(d2, d0), (prec, rep)
+    assert S.get_tuning("graphs") == (0 if resident else 2)  # one a precision, captured once
     S.close()
 
 
@@ -206,11 +217,13 @@ def test_vcycle_on_a_block_diagonal_batch_matches_oracle():
     S.close()
 
 
+@pytest.mark.parametrize("fp32_rows", [700000, 0])
 @pytest.mark.parametrize("case", ["tet_grf_16", "p2_blocks_64"])
-def test_nested_pcg_matches_per_level_pcg(oracle, case):
+def test_nested_pcg_matches_per_level_pcg(oracle, case, fp32_rows):
     """The nested-ordered PCG (standard CG, reductions folded into the next
     kernel) and the per-level pipelined PCG: both reach the FP64 target, in
-    FP64 and with FP32 inner solves under FP64 refinement; with the V-cycle
+    FP64 and with FP32 inner solves under FP64 refinement (amg_fp32_rows 0),
+    the nested V-cycle in FP64 in one launch and by launches; with the V-cycle
     (amg_wcycle 0) their iteration counts are within 20% of each other, and
     the W-cycle kernel takes no more iterations than the V-cycle."""
     from feng_amd.api import FN_CONST, FN_ELEM, PC_AMG, PREC_FP32_IR, Fn, Mesh
@@ -227,21 +240,27 @@ def test_nested_pcg_matches_per_level_pcg(oracle, case):
     ia, ja = S.get_csr()
     val, rhs = S.get_system()
     out = {}
-    for kern in (2, 1, 3):  # 3: nested with the V-cycle
-        S.set_tuning("amg_kernel", 2 if kern == 3 else kern)
-        S.set_tuning("amg_wcycle", 0 if kern == 3 else 1)
+    S.set_tuning("amg_fp32_rows", fp32_rows)
+    for kern in (2, 1, 3, 4):  # 3: nested with the V-cycle, 4: the same by launches
+        S.set_tuning("amg_kernel", 2 if kern >= 3 else kern)
+        S.set_tuning("amg_wcycle", 0 if kern >= 3 else 1)
+        S.set_tuning("resident", int(kern != 4))
         for prec in (0, PREC_FP32_IR):
             r, du = S.solve(pc=PC_AMG, precision=prec, rtol=1e-8, inner_rtol=1e-4, want_du=True)
             assert r.converged and r.relres <= 1e-8, (kern, prec, r)
             res = rhs - oracle.spmv(ia, ja, val, du)
             assert np.linalg.norm(res) <= 1.01e-8 * np.linalg.norm(rhs), (kern, prec)
+            one = kern == 3 and (prec == 0 or fp32_rows > 0)
+            assert S.get_tuning("resident_ran") == one
+            assert prec == 0 or fp32_rows > 0 or r.outer_iterations >= 2, (kern, r)
             out[(kern, prec)] = (r.iterations, du)
     for prec in (0, PREC_FP32_IR):
         itW, it1, itV = out[(2, prec)][0], out[(1, prec)][0], out[(3, prec)][0]
         print(case, "precision", prec, "iterations nested W / per-level / nested V:", itW, it1, itV, flush=True)
         assert abs(itV - it1) <= max(2, 0.2 * it1), (prec, itV, it1)
         assert itW <= itV + 1, (prec, itW, itV)
-        for kern in (2, 3):
+        assert abs(out[(4, prec)][0] - itV) <= 2, (prec, itV)
+        for kern in (2, 3, 4):
             d2, d1 = out[(kern, prec)][1], out[(1, prec)][1]
             assert np.abs(d2 - d1).max() <= 1e-5 * np.abs(d1).max()
     S.close()

@@ -87,7 +87,23 @@ def test_fp32_refinement_reaches_fp64_tolerance(oracle):
     S, num = diffusion_system(m, 2, 2, _fn((0, 1.0, 0.0, None)), _fn((1, -2 * math.pi ** 2, 0.0, None)))
     S.assemble(3, PREC_FP32_IR)
     r = S.solve(precision=PREC_FP32_IR, rtol=1e-10)
-    assert r.converged and r.relres <= 1e-10 and r.outer_iterations >= 2
+    assert r.converged and r.relres <= 1e-10 and S.get_tuning("resident_ran") == 1  # FP64, in one launch
+    S.set_tuning("resident", 0)
+    for pipe in (2, 1, 0):  # FP32 inner solves: Chronopoulos-Gear, tiled, Chronopoulos-Gear
+        S.set_tuning("pipe_kernel", pipe)
+        r = S.solve(precision=PREC_FP32_IR, rtol=1e-10)
+        assert r.converged and r.relres <= 1e-10 and r.outer_iterations >= 2
+    # FP32 values that are no longer the matrix's: the first correction is rejected, FP64 inner solves finish
+    val, rhs = S.get_system()
+    S.set_system(val=3.0 * val, rhs=rhs)
+    for pipe in (2, 1, 0):
+        S.set_tuning("pipe_kernel", pipe)
+        r, x = S.solve(precision=PREC_FP32_IR, rtol=1e-10, want_du=True)
+        assert r.converged and r.relres <= 1e-10 and r.outer_iterations >= 2
+        ia, ja = S.get_csr()
+        res = rhs - oracle.spmv(ia, ja, 3.0 * val, x)
+        assert np.linalg.norm(res) <= 1.01e-10 * np.linalg.norm(rhs)
+    S.set_system(val=val, rhs=rhs)
     r64 = S.solve(rtol=1e-10)
     assert r64.converged
     S.close()
@@ -150,12 +166,15 @@ def test_fp32_mfma_element_matrices(kind, deg):
     v64, r64 = S.get_system()
     r = S.solve(precision=PREC_FP32_IR, rtol=1e-10)
     assert r.converged and r.relres <= 1e-10
+    S.set_tuning("resident", 0)  # FP32 inner solves from here on
+    r = S.solve(precision=PREC_FP32_IR, rtol=1e-10)
+    assert r.converged and r.relres <= 1e-10 and r.outer_iterations >= 2
     # the FP32 values themselves: solve with them must reach the FP64 target
     S.set_tuning("fp32_values", 0)
     S.setToZero()
     S.assemble(3, PREC_FP32_IR)
     r0 = S.solve(precision=PREC_FP32_IR, rtol=1e-10)
-    assert r0.converged
+    assert r0.converged and r0.outer_iterations >= 2
     S.close()
 
 

@@ -186,14 +186,17 @@ def test_fp32_values_and_solution_vs_fp64_oracle(oracle, name):
     S.setToZero()
     S.assemble(3, PREC_FP32_IR)
     rtol = 1e-8 if kind == 4 else 1e-10
-    r, du = S.solve(precision=PREC_FP32_IR, rtol=rtol, want_du=True)
-    assert r.converged and r.relres <= rtol
-    res = rhs0 - oracle.spmv(ia0, ja0, val0, du)
-    assert np.linalg.norm(res) <= 1.01 * rtol * np.linalg.norm(rhs0)
+    # (resident 0; in one launch the iteration is FP64)
     x0, _, _ = oracle.cg_jacobi(ia0, ja0, val0, rhs0, rtol * 0.1, 40000)
-    err_x = np.abs(du - x0).max() / np.abs(x0).max()
-    print(name, f"FP32-refined solution vs FP64 oracle CG: {err_x:.2e}", flush=True)
-    assert err_x <= 1e-5
+    for resident in (1, 0):
+        S.set_tuning("resident", resident)
+        r, du = S.solve(precision=PREC_FP32_IR, rtol=rtol, want_du=True)
+        assert r.converged and r.relres <= rtol and (resident or r.outer_iterations >= 2)
+        res = rhs0 - oracle.spmv(ia0, ja0, val0, du)
+        assert np.linalg.norm(res) <= 1.01 * rtol * np.linalg.norm(rhs0)
+        err_x = np.abs(du - x0).max() / np.abs(x0).max()
+        print(name, resident, f"FP32-refined solution vs FP64 oracle CG: {err_x:.2e}", flush=True)
+        assert err_x <= 1e-5
     S.close()
 
 

@@ -127,6 +127,11 @@ def test_learned_pcg_converges_in_fp64_and_fp32():
     S.assemble(3, PREC_FP32_IR)
     r2 = S.solve(pc=PC_LEARNED, precision=PREC_FP32_IR, rtol=1e-8)
     assert r2.converged and r2.relres <= 1e-8
+    S.set_tuning("resident", 0)  # FP32 inner solves, FP64 iteration, by launches
+    r2 = S.solve(pc=PC_LEARNED, precision=PREC_FP32_IR, rtol=1e-8)
+    assert r2.converged and r2.relres <= 1e-8 and r2.outer_iterations >= 2
+    r2 = S.solve(pc=PC_LEARNED, rtol=1e-8)
+    assert r2.converged and r2.relres <= 1e-8
     r3 = S.solve(pc=PC_IC0, rtol=1e-8)
     assert r3.converged
     S.close()

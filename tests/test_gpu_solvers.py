@@ -54,6 +54,13 @@ def test_split_ic0_pcg_beats_jacobi(oracle):
     ri32 = S.solve(pc=PC_IC0, precision=PREC_FP32_IR, rtol=1e-8, inner_rtol=1e-2)
     assert rj.converged and ri.converged and ri32.converged
     assert ri.iterations < 0.7 * rj.iterations
+    # by launches: FP32 inner solves, tiled (pipe_kernel 1) and not, and the FP64 forms
+    S.set_tuning("resident", 0)
+    for pipe in (2, 1, 0):
+        S.set_tuning("pipe_kernel", pipe)
+        r64 = S.solve(pc=PC_IC0, rtol=1e-8)
+        r32 = S.solve(pc=PC_IC0, precision=PREC_FP32_IR, rtol=1e-8, inner_rtol=1e-2)
+        assert r64.converged and r32.converged and r32.outer_iterations >= 2 and r64.iterations < 0.7 * rj.iterations
     ia, ja = S.get_csr()
     val, rhs = S.get_system()
     res = rhs - oracle.spmv(ia, ja, val, du)

@@ -633,7 +633,8 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
         bn = rn;
         target = resUniform(fmax(a.rtol * bn, a.atol));
         tol2 = resUniform(0.25 * target * target);
-        if(bn == 0.) reason = 2;
+        if(bn == 0. || rn <= target) reason = 2;
+        else if(a.maxit <= 0) reason = -3;
       } else {
         if(rn <= target) reason = 2;
         else if(!(rn == rn)) reason = -9;

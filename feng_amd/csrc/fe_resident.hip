@@ -75,6 +75,7 @@ struct ResArgs {
   double *maxima;
   double rtol, atol, dtol;
   int maxit;
+  int refine;      // FE_PREC_FP32_IR: the targets are tested before the first iteration too, as that loop does
   long long wait;  // ticks
 };
 
@@ -340,10 +341,10 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
         bn = rn;
         target = resUniform(fmax(a.rtol * bn, a.atol));
         tol2 = resUniform(target * target * 0.25);
-        if(bn == 0.) {
-          reason = 2;
-          break;
-        }
+        if(bn == 0.) reason = 2;
+        else if(a.refine && rn <= target) reason = 2;
+        else if(a.refine && a.maxit <= 0) reason = -3;
+        if(reason) break;
       } else {
         if(rn <= target) reason = 2;
         else if(code == 4 || !(rn == rn)) reason = -9;
@@ -646,7 +647,8 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
         bn = rn;
         target = resUniform(fmax(a.rtol * bn, a.atol));
         tol2 = resUniform(target * target * 0.25);
-        if(bn == 0.) reason = 2;
+        if(bn == 0. || rn <= target) reason = 2;
+        else if(a.maxit <= 0) reason = -3;
       } else {
         if(rn <= target) reason = 2;
         else if(code == 4 || !(rn == rn)) reason = -9;
@@ -849,7 +851,7 @@ ResArgs resArgs(const fe_hip_ctx *ctx, const FeResident &R, const fe_hip_solver_
   const int hcap = std::min(kResH, kResLds / 16 - R.RW);
   return ResArgs{ctx->n,   R.G,        R.RW, R.H, hcap,    ctx->d_ia, ctx->d_ja,       ctx->d_val, R.d_idx, R.d_hcol,
                  R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter,
-                 resWaitTicks(ctx)};
+                 o->precision == FE_PREC_FP32_IR, resWaitTicks(ctx)};
 }
 
 }  // namespace

@@ -159,3 +159,29 @@ def test_resident_split_equals_launch_per_iteration(kind, N, pc):
     rz, xz = S.solve(pc=pcn, want_du=True)
     assert rz.converged and rz.iterations == 0 and not xz.any()
     S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0", "amg"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_a_target_above_the_right_hand_side_takes_no_iteration(pc, prec):
+    """atol above ||b||: the zero correction is the answer of the multigrid, the
+    split and the refined solves (FP64 Jacobi-PCG aims at half the target and
+    iterates), and no budget is none; both as by launches."""
+    from feng_amd.api import PC_AMG, PC_IC0, PC_JACOBI, PREC_FP32_IR
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0, "amg": PC_AMG}[pc]
+    S, _ = _system(4, 12)
+    S.setToZero()
+    S.assemble(3, PREC_FP32_IR)
+    bn = np.linalg.norm(S.get_system()[1])
+    for opts in (dict(atol=1.5 * bn), dict(atol=20.0 * bn), dict(max_iter=0)):
+        out = []
+        for resident in (0, 1):
+            S.set_tuning("resident", resident)
+            r, x = S.solve(pc=pcn, precision=prec, want_du=True, **opts)
+            assert S.get_tuning("resident_ran") == resident
+            out.append((r.iterations, r.outer_iterations, r.converged, r.reason, r.norm_rhs_inf))
+            if (pc, prec) != ("jacobi", 0):
+                assert out[-1][:4] == ((0, 0, False, -3) if "max_iter" in opts else (0, 0, True, 2))
+                assert r.relres == 1.0 and not x.any() and r.norm_axb_inf == r.norm_rhs_inf
+        assert out[0] == out[1], (opts, out)
+    S.close()

@@ -1181,7 +1181,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
   res->reason = out.reason;
   res->iters = out.iters;
   res->outer = out.outer;
-  res->relres = out.bn > 0. ? out.rn / out.bn : 0.;
+  res->relres = out.bn == 0. ? 0. : out.rn / out.bn;  // not a number stays that
   const double *mx = (const double *)(R.h_out + 1);
   for(int k = 0; k < 3; ++k) res->inf[k] = 0.;
   for(int k = 0; k < 3 * a.G; ++k) res->inf[k % 3] = std::max(res->inf[k % 3], mx[k]);

@@ -185,3 +185,19 @@ def test_a_target_above_the_right_hand_side_takes_no_iteration(pc, prec):
                 assert r.relres == 1.0 and not x.any() and r.norm_axb_inf == r.norm_rhs_inf
         assert out[0] == out[1], (opts, out)
     S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0", "amg"])
+def test_a_right_hand_side_that_is_not_a_number_is_reported(pc):
+    from feng_amd.api import PC_AMG, PC_IC0, PC_JACOBI
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0, "amg": PC_AMG}[pc]
+    S, _ = _system(4, 12)
+    rhs = S.get_system()[1]
+    rhs[3] = np.nan
+    S.set_system(rhs=rhs)
+    for resident in (0, 1):
+        S.set_tuning("resident", resident)
+        r = S.solve(pc=pcn, max_iter=50)
+        assert S.get_tuning("resident_ran") == resident
+        assert not r.converged and r.reason == -9 and np.isnan(r.relres)
+    S.close()

@@ -68,7 +68,7 @@ constexpr int kSentBit = 0x8000;
 constexpr int kSets = 3;          // sets of exchange slots
 
 struct ArOut {
-  int reason, iters, outer, gaveUp, badPivot, pad;
+  int reason, iters, outer, gaveUp, badPivot, ended;
   double bn, rn;
 };
 
@@ -638,8 +638,10 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
       } else {
         if(rn <= target) reason = 2;
         else if(!(rn == rn)) reason = -9;
-        else if(it >= a.maxit || breakdowns > 20) reason = -3;
+        else if(breakdowns > 20) reason = -3;
         else if(rn / bn > a.dtol) reason = -4;
+        else if(outer >= kResOuter) reason = kResLimit;
+        else if(it >= a.maxit) reason = -3;
       }
       if(reason) break;
 #pragma unroll
@@ -775,7 +777,8 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
   if(t == 0) {
     if(gaveUp) __hip_atomic_store(&a.out->gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if(wg == 0) {
-      a.out->reason = reason;
+      a.out->ended = 1;
+      a.out->reason = reason == kResLimit ? 0 : reason;
       a.out->iters = it;
       a.out->outer = outer;
       a.out->badPivot = *a.badPivot;
@@ -1171,7 +1174,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
     return FE_STATUS_OK;
   }
   const ArOut &out = *R.h_out;
-  if(out.gaveUp || out.reason == 0) {  // a wait ran out: the other kernels take over
+  if(out.gaveUp || !out.ended) {  // a wait ran out: the other kernels take over
     ctx->iterTimer.used = 0;
     ctx->residentGaveUp = true;
     return FE_STATUS_OK;

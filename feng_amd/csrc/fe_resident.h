@@ -34,6 +34,12 @@ namespace fe_res {
 
 constexpr unsigned long long kSentinel = 0x7FF4DEAD5EA7F00Dull;
 constexpr int kResBufs = 4;
+// Most solves from a true residual (the launch-per-iteration loops of refined,
+// split and multigrid solves have the same bound); a target below the floor of
+// FP64 would otherwise be tried until the iteration budget ends.  A solve that
+// stops there has no reason code (0): kResLimit inside a kernel.
+constexpr int kResOuter = 60;
+constexpr int kResLimit = 100;
 
 __device__ __forceinline__ unsigned long long resLoad(const unsigned long long *p)
 {

@@ -39,7 +39,7 @@ using namespace fe_res;
 // What a solve returns to the host, and per workgroup the largest |x|, |b|,
 // |b - A x| of its rows behind it.
 struct ResOut {
-  int reason, iters, outer, gaveUp;
+  int reason, iters, outer, gaveUp, ended, pad;
   double bn, rn;
 };
 
@@ -75,7 +75,8 @@ struct ResArgs {
   double *maxima;
   double rtol, atol, dtol;
   int maxit;
-  int refine;      // FE_PREC_FP32_IR: the targets are tested before the first iteration too, as that loop does
+  int refine;      // FE_PREC_FP32_IR: the targets are tested before the first iteration too, with a bound on
+                   // the restarts, as in that loop
   long long wait;  // ticks
 };
 
@@ -158,7 +159,7 @@ __global__ void resFill(size_t count, unsigned long long *__restrict__ buf, ResO
 {
   for(size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
     buf[i] = kSentinel;
-  if(blockIdx.x == 0 && threadIdx.x == 0) *out = ResOut{0, 0, 0, 0, 0., 0.};
+  if(blockIdx.x == 0 && threadIdx.x == 0) *out = ResOut{0, 0, 0, 0, 0, 0, 0., 0.};
 }
 
 // The workgroup's largest |x|, |b|, |b - A x|.
@@ -348,13 +349,16 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
       } else {
         if(rn <= target) reason = 2;
         else if(code == 4 || !(rn == rn)) reason = -9;
-        else if(it >= a.maxit) reason = -3;
+        else if(it >= a.maxit && !a.refine) reason = -3;
         else if(rn / bn > a.dtol) reason = -4;
         else if(code == 3 && ++breakdowns > 20) reason = -3;
+        else if(a.refine && outer >= kResOuter) reason = kResLimit;
+        else if(it >= a.maxit) reason = -3;
         if(reason) break;
         // again from the true residual: after a breakdown, or when the
-        // recursive residual met a target the true one has not (aim lower)
-        if(code != 3) tol2 = resUniform(0.01 * tol2);
+        // recursive residual met a target the true one has not (aim lower; the
+        // bounded restarts of a refined solve keep the target)
+        if(code != 3 && !a.refine) tol2 = resUniform(0.01 * tol2);
         code = 0;
       }
       s = z = p = 0.;
@@ -397,7 +401,8 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
   if(t == 0) {
     if(gaveUp) __hip_atomic_store(&a.out->gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if(wg == 0) {
-      a.out->reason = reason;
+      a.out->ended = 1;
+      a.out->reason = reason == kResLimit ? 0 : reason;
       a.out->iters = it;
       a.out->outer = outer;
       a.out->bn = bn;
@@ -652,9 +657,10 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
       } else {
         if(rn <= target) reason = 2;
         else if(code == 4 || !(rn == rn)) reason = -9;
-        else if(it >= a.maxit) reason = -3;
-        else if(rn / bn > a.dtol) reason = -4;
         else if(code == 3 && ++breakdowns > 20) reason = -3;
+        else if(rn / bn > a.dtol) reason = -4;
+        else if(outer >= kResOuter) reason = kResLimit;
+        else if(it >= a.maxit) reason = -3;
         code = 0;  // again from the true residual
       }
       if(reason) break;
@@ -707,7 +713,8 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
   if(t == 0) {
     if(gaveUp) __hip_atomic_store(&a.out->gaveUp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if(wg == 0) {
-      a.out->reason = reason;
+      a.out->ended = 1;
+      a.out->reason = reason == kResLimit ? 0 : reason;
       a.out->iters = it;
       a.out->outer = outer;
       a.out->bn = bn;
@@ -814,7 +821,7 @@ int resRun(fe_hip_ctx *ctx, FeResident &R, unsigned long long *buf, size_t cells
     return FE_STATUS_OK;
   }
   const ResOut &out = *R.h_out;
-  if(out.gaveUp || out.reason == 0) {  // a wait ran out: the other kernels take over
+  if(out.gaveUp || !out.ended) {  // a wait ran out: the other kernels take over
     ctx->spmvTimer.used = 0;
     ctx->residentGaveUp = true;
     return FE_STATUS_OK;

@@ -201,3 +201,28 @@ def test_a_right_hand_side_that_is_not_a_number_is_reported(pc):
         assert S.get_tuning("resident_ran") == resident
         assert not r.converged and r.reason == -9 and np.isnan(r.relres)
     S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0", "amg"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_a_target_below_the_floor_ends_after_the_same_restarts(pc, prec):
+    """60 solves from a true residual at most, and then no reason code, as by
+    launches; FP64 Jacobi-PCG has no such bound and ends with the budget or
+    after 20 breakdowns of the recurrences."""
+    from feng_amd.api import PC_AMG, PC_IC0, PC_JACOBI, PREC_FP32_IR
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0, "amg": PC_AMG}[pc]
+    S, _ = _system(4, 12)
+    S.setToZero()
+    S.assemble(3, PREC_FP32_IR)
+    out = []
+    for resident in (0, 1):
+        S.set_tuning("resident", resident)
+        r, x = S.solve(pc=pcn, precision=prec, rtol=1e-17, max_iter=3000, want_du=True)
+        assert S.get_tuning("resident_ran") == resident
+        out.append(r)
+        assert not r.converged and r.relres < 1e-14
+        if (pc, prec) == ("jacobi", 0):
+            assert r.reason == -3
+        else:
+            assert r.reason == 0 and r.outer_iterations == 60 and r.iterations < 3000
+    S.close()

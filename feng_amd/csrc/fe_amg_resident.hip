@@ -1139,7 +1139,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
   a.atol = o->atol;
   a.dtol = o->dtol;
   a.oc = ctx->amgOverCorrect;
-  a.maxit = o->max_iter;
+  a.maxit = std::min(o->max_iter, ctx->residentMaxIter);
   a.wait = resWaitTicks(ctx);
   bool fits = false;
   {
@@ -1177,6 +1177,10 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
   if(out.gaveUp || !out.ended) {  // a wait ran out: the other kernels take over
     ctx->iterTimer.used = 0;
     ctx->residentGaveUp = true;
+    return FE_STATUS_OK;
+  }
+  if(resCutShort(ctx, o, out.iters, out.reason)) {
+    ctx->iterTimer.used = 0;
     return FE_STATUS_OK;
   }
   FE_REQUIRE(ctx, out.bn == 0. || !out.badPivot, "AMG: the coarsest operator is not positive definite");

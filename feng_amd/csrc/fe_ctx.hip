@@ -761,6 +761,9 @@ int fe_hip_set_tuning(fe_hip_ctx *ctx, const char *key, int value)
   } else if(k == "resident_wait_us") {
     FE_REQUIRE(ctx, value >= 0 && value <= 1000000, "resident_wait_us must be in [0, 1000000]");
     ctx->residentWaitUs = value;
+  } else if(k == "resident_max_iter") {
+    FE_REQUIRE(ctx, value >= 1, "resident_max_iter must be >= 1");
+    ctx->residentMaxIter = value;
   } else if(k == "ilu_sweeps") {
     FE_REQUIRE(ctx, value >= 0 && value <= 64,
                "ilu_sweeps must be 0 (exact triangular solves) or a sweep count in [1, 64]");
@@ -858,6 +861,7 @@ int fe_hip_get_tuning(fe_hip_ctx *ctx, const char *key, int *value)
   else if(k == "resident") *value = ctx->resident;
   else if(k == "amg_fp32_rows") *value = ctx->amgFp32Rows;
   else if(k == "resident_wait_us") *value = ctx->residentWaitUs;
+  else if(k == "resident_max_iter") *value = ctx->residentMaxIter;
   else if(k == "resident_ran") *value = ctx->residentRan;
   else if(k == "resident_gave_up") *value = ctx->residentGaveUp;
   else if(k == "gmres_orth") *value = ctx->gmresOrth;

@@ -208,6 +208,7 @@ struct fe_hip_ctx {
   int amgFp32Rows = 700000;     // multigrid-PCG at FE_PREC_FP32_IR: FP32 iterations above this many rows, FP64 ones up to it
   int resident = 1;             // CG: all iterations in one launch where the system fits (0: never)
   int residentWaitUs = 50000;   // longest wait of such a launch for another workgroup's value
+  int residentMaxIter = 100000;  // most iterations of such a launch (0.3 to 2 s: nothing can interrupt it)
   bool residentRan = false;     // the last solve was one
   bool residentGaveUp = false;  // a wait ran out: the other kernels until the tuning key `resident` is set again
 

@@ -63,6 +63,13 @@ inline long long resWaitTicks(const fe_hip_ctx *ctx)
   return ctx->residentWaitUs > 0 ? 100ll * ctx->residentWaitUs : -1;
 }
 
+// A solve that the iteration limit of a launch has cut short of its own budget:
+// the launches per iteration repeat it.
+inline bool resCutShort(const fe_hip_ctx *ctx, const fe_hip_solver_opts *o, int iters, int reason)
+{
+  return o->max_iter > ctx->residentMaxIter && iters >= ctx->residentMaxIter && reason != 2;
+}
+
 // Polls the K slots base[idx[k]] (idx < 0: none) until all have arrived; false
 // when the time is up.  The loads of a round are issued together.
 template <int K>

@@ -797,7 +797,8 @@ namespace {
 // One resident launch over `bufLen` slots, and what it returned.  launch(&fits)
 // enqueues the kernel.
 template <typename F>
-int resRun(fe_hip_ctx *ctx, FeResident &R, unsigned long long *buf, size_t cells, FeResidentResult *res, F launch)
+int resRun(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, FeResident &R, unsigned long long *buf, size_t cells,
+           FeResidentResult *res, F launch)
 {
   bool fits = false;
   {
@@ -824,6 +825,10 @@ int resRun(fe_hip_ctx *ctx, FeResident &R, unsigned long long *buf, size_t cells
   if(out.gaveUp || !out.ended) {  // a wait ran out: the other kernels take over
     ctx->spmvTimer.used = 0;
     ctx->residentGaveUp = true;
+    return FE_STATUS_OK;
+  }
+  if(resCutShort(ctx, o, out.iters, out.reason)) {
+    ctx->spmvTimer.used = 0;
     return FE_STATUS_OK;
   }
   res->ran = ctx->residentRan = true;
@@ -857,8 +862,8 @@ ResArgs resArgs(const fe_hip_ctx *ctx, const FeResident &R, const fe_hip_solver_
 {
   const int hcap = std::min(kResH, kResLds / 16 - R.RW);
   return ResArgs{ctx->n,   R.G,        R.RW, R.H, hcap,    ctx->d_ia, ctx->d_ja,       ctx->d_val, R.d_idx, R.d_hcol,
-                 R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol, o->max_iter,
-                 o->precision == FE_PREC_FP32_IR, resWaitTicks(ctx)};
+                 R.d_hcnt, ctx->d_rhs, x,    buf, R.d_out, (double *)(R.d_out + 1), o->rtol, o->atol, o->dtol,
+                 std::min(o->max_iter, ctx->residentMaxIter), o->precision == FE_PREC_FP32_IR, resWaitTicks(ctx)};
 }
 
 }  // namespace
@@ -872,7 +877,7 @@ int feResidentJacobi(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, Fe
   if(!R.usable) return FE_STATUS_OK;
   const ResArgs a = resArgs(ctx, R, o, x, R.d_buf);
   const size_t lds = 2 * (size_t)(R.RW + R.H) * sizeof(double);
-  return resRun(ctx, R, R.d_buf, kResBufs * ((size_t)ctx->n + 3 * (size_t)R.G), res, [&](bool *fits) {
+  return resRun(ctx, o, R, R.d_buf, kResBufs * ((size_t)ctx->n + 3 * (size_t)R.G), res, [&](bool *fits) {
     auto *const k = R.TB == 512 ? (R.E == 8 ? resJacobi<512, 8> : R.E == 16 ? resJacobi<512, 16> : resJacobi<512, 24>)
                                 : (R.E == 8 ? resJacobi<1024, 8> : R.E == 16 ? resJacobi<1024, 16> : resJacobi<1024, 24>);
     return launchRes(ctx, k, R.TB, R, a, lds, fits);
@@ -905,7 +910,7 @@ int feResidentSplit(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, FeR
   }
   const SplitArgs a{resArgs(ctx, R, o, x, R.d_splitBuf), R.d_pos, P.d_gL32, P.d_gU32, P.d_dinv32};
   const size_t lds = 2 * (size_t)(R.RW + R.H) * sizeof(double);
-  return resRun(ctx, R, R.d_splitBuf, cells, res, [&](bool *fits) {
+  return resRun(ctx, o, R, R.d_splitBuf, cells, res, [&](bool *fits) {
     auto *const k = R.TB == 512 ? (R.E == 8 ? resSplit<512, 8> : R.E == 16 ? resSplit<512, 16> : resSplit<512, 24>)
                                 : (R.E == 8 ? resSplit<1024, 8> : resSplit<1024, 16>);
     return launchRes(ctx, k, R.TB, R, a, lds, fits);

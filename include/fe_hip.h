@@ -271,7 +271,9 @@ int fe_hip_set_profiling(fe_hip_ctx *ctx, int on);
  * default: CG solves of systems that fit in one launch; setting it clears
  * "resident_gave_up"),
  * "resident_wait_us" (longest wait of such a launch, default 50000; when one
- * runs out the solve is repeated by launches, and later solves take them too).
+ * runs out the solve is repeated by launches, and later solves take them too),
+ * "resident_max_iter" (most iterations of such a launch, default 100000; a
+ * solve that needs more is repeated by launches).
  * Read-only: "resident_ran" (the last solve was one launch),
  * "resident_gave_up" (a wait has run out), "graphs" (captured graphs the
  * context holds). */

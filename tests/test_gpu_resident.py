@@ -226,3 +226,25 @@ def test_a_target_below_the_floor_ends_after_the_same_restarts(pc, prec):
         else:
             assert r.reason == 0 and r.outer_iterations == 60 and r.iterations < 3000
     S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0", "amg"])
+def test_a_launch_has_a_bounded_length(pc):
+    """A solve that needs more iterations than one launch may take is the
+    launch-per-iteration one; a budget within the limit is not affected."""
+    from feng_amd.api import PC_AMG, PC_IC0, PC_JACOBI
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0, "amg": PC_AMG}[pc]
+    S, _ = _system(4, 12)
+    S.set_tuning("resident", 0)
+    r0, x0 = S.solve(pc=pcn, rtol=1e-9, want_du=True)
+    S.set_tuning("resident", 1)
+    S.set_tuning("resident_max_iter", r0.iterations // 2)
+    r1, x1 = S.solve(pc=pcn, rtol=1e-9, want_du=True)
+    assert S.get_tuning("resident_ran") == 0 and S.get_tuning("resident_gave_up") == 0
+    assert r1.converged and r1.iterations == r0.iterations and np.array_equal(x1, x0)
+    r2 = S.solve(pc=pcn, rtol=1e-9, max_iter=r0.iterations // 2)
+    assert S.get_tuning("resident_ran") == 1 and r2.reason == -3 and r2.iterations == r0.iterations // 2
+    S.set_tuning("resident_max_iter", r0.iterations + 10)
+    r3 = S.solve(pc=pcn, rtol=1e-9)
+    assert S.get_tuning("resident_ran") == 1 and r3.converged
+    S.close()

@@ -1755,9 +1755,10 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   // solves (FE_PREC_FP32_IR) take the FP64 launch too: exchanges bound it, and
   // restarts from the true residual cost iterations.  Jacobi, P1 tetrahedra
   // 64^3: FP32 11.6 ms (552 iterations), here 2.7 (422); learned factor 45^3:
-  // 5.7 ms (162), here 1.7 (121).
-  if((!split && tiled64 && (o->precision == FE_PREC_FP64 || ctx->d_val32)) ||
-     (amg && o->precision == FE_PREC_FP64)) {
+  // 5.7 ms (162), here 1.7 (121).  A pipe_kernel that names another kernel is
+  // taken at its word.
+  const bool oneLaunch = o->precision == FE_PREC_FP64 ? amg || tiled64 : !amg && ctx->pipeKernel == 2 && ctx->d_val32;
+  if(oneLaunch && (!split || amg)) {
     FeResidentResult R;
     R.ran = false;
     if(!amg) {
@@ -1836,7 +1837,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   }
 
   FeResidentResult one{};
-  if(split && !amg && bn != 0. && (o->precision == FE_PREC_FP64 || ctx->d_val32))
+  if(oneLaunch && split && !amg && bn != 0.)
     if(int rc = feResidentSplit(ctx, o, ctx->d_du, &one)) return rc;
   const bool nested = amg && feAmgNestedUsable(ctx);
   if(bn == 0.) {

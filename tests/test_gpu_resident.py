@@ -248,3 +248,26 @@ def test_a_launch_has_a_bounded_length(pc):
     r3 = S.solve(pc=pcn, rtol=1e-9)
     assert S.get_tuning("resident_ran") == 1 and r3.converged
     S.close()
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "ic0"])
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("pipe", [0, 1, 2])
+def test_pipe_kernel_picks_the_kernel(pc, prec, pipe):
+    """One launch stands in for the tiled FP64 kernels and for the default choice
+    at FE_PREC_FP32_IR; the kernels that pipe_kernel names otherwise run."""
+    from feng_amd.api import PC_IC0, PC_JACOBI, PREC_FP32_IR
+    pcn = {"jacobi": PC_JACOBI, "ic0": PC_IC0}[pc]
+    S, _ = _system(4, 12)
+    S.setToZero()
+    S.assemble(3, PREC_FP32_IR)
+    S.set_tuning("pipe_kernel", pipe)
+    out = []
+    for resident in (0, 1):
+        S.set_tuning("resident", resident)
+        out.append(S.solve(pc=pcn, precision=prec, rtol=1e-9, want_du=True))
+    one = pipe == 2 or (pipe == 1 and prec == 0)
+    assert S.get_tuning("resident_ran") == one
+    assert out[0][0].converged and out[1][0].converged
+    assert np.array_equal(out[0][1], out[1][1]) == (not one)
+    S.close()

@@ -24,6 +24,7 @@
 #include "fe_tile.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -1757,6 +1758,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   // 64^3: FP32 11.6 ms (552 iterations), here 2.7 (422); learned factor 45^3:
   // 5.7 ms (162), here 1.7 (121).  A pipe_kernel that names another kernel is
   // taken at its word.
+  double setupMs = 0.;
   const bool oneLaunch = o->precision == FE_PREC_FP64 ? amg || tiled64 : !amg && ctx->pipeKernel == 2 && ctx->d_val32;
   if(oneLaunch && (!split || amg)) {
     FeResidentResult R;
@@ -1764,7 +1766,9 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
     if(!amg) {
       if(int rc = feResidentJacobi(ctx, o, ctx->d_du, &R)) return rc;
     } else {
+      const auto s0 = std::chrono::steady_clock::now();
       if(int rc = feAmgSetup(ctx)) return rc;
+      setupMs = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - s0).count();
       if(feAmgNestedUsable(ctx))
         if(int rc = feAmgResidentSolve(ctx, o, ctx->d_du, &R)) return rc;
     }
@@ -1786,6 +1790,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
         stats->norm_rhs_inf = R.inf[1];
         stats->norm_axb_inf = R.inf[2];
         stats->ms_solve = ms;
+        stats->ms_setup = setupMs;
       }
       if(du) {
         FE_HIP_TRY(ctx, hipMemcpyAsync(du, ctx->d_du, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
@@ -1806,7 +1811,6 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   int iters = 0, outer = 0, converged = 0, reason = 0, done = 0, breakdowns = 0;
   double relres = bn > 0. ? 1. : 0.;
 
-  double setupMs = 0.;
   if(split && bn != 0.) {
     hipEvent_t s0, s1;
     FE_HIP_TRY(ctx, hipEventCreate(&s0));
@@ -1826,7 +1830,7 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
     FE_HIP_TRY(ctx, hipEventSynchronize(s1));
     float sm = 0.f;
     FE_HIP_TRY(ctx, hipEventElapsedTime(&sm, s0, s1));
-    setupMs = sm;
+    setupMs += sm;
     (void)hipEventDestroy(s0);
     (void)hipEventDestroy(s1);
     FePrecond &P = ctx->pc;

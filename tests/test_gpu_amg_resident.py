@@ -98,3 +98,16 @@ def test_fp32_multigrid_runs_the_fp64_iteration(kernel, resident):
     assert r0.converged and r1.iterations == r0.iterations and r1.outer_iterations == r0.outer_iterations
     assert np.array_equal(d0, d1)
     S.close()
+
+
+@pytest.mark.parametrize("resident", [0, 1])
+def test_set_up_time_is_reported(resident):
+    """ms_setup: the hierarchy of the first solve (some milliseconds of host
+    work); next to nothing on later ones."""
+    from feng_amd.api import PC_AMG
+    S, _ = _system(4, 24)
+    S.set_tuning("resident", resident)
+    first, second = S.solve(pc=PC_AMG), S.solve(pc=PC_AMG)
+    assert S.get_tuning("resident_ran") == resident
+    assert first.ms_setup > 0.3 and first.ms_setup > 5 * second.ms_setup and first.ms_setup < first.ms_solve
+    S.close()

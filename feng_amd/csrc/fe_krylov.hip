@@ -1758,7 +1758,17 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
   // 64^3: FP32 11.6 ms (552 iterations), here 2.7 (422); learned factor 45^3:
   // 5.7 ms (162), here 1.7 (121).  A pipe_kernel that names another kernel is
   // taken at its word.
-  double setupMs = 0.;
+  double setupMs = 0., bn = -1.;  // ||rhs||, not known yet
+  auto rhsNorm = [&]() -> int {
+    double bb = 0.;
+    hipLaunchKernelGGL(sumSquares, dim3(kGrid), dim3(kTB), 0, ctx->stream, n, ctx->d_rhs, w.part);
+    hipLaunchKernelGGL(finalizeSums, dim3(1), dim3(kTB), 0, ctx->stream, w.part, kGrid, 1, w.res + 8);
+    FE_HIP_TRY(ctx, hipGetLastError());
+    FE_HIP_TRY(ctx, hipMemcpyAsync(&bb, w.res + 8, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    bn = std::sqrt(bb);
+    return FE_STATUS_OK;
+  };
   const bool oneLaunch = o->precision == FE_PREC_FP64 ? amg || tiled64 : !amg && ctx->pipeKernel == 2 && ctx->d_val32;
   if(oneLaunch && (!split || amg)) {
     FeResidentResult R;
@@ -1766,10 +1776,14 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
     if(!amg) {
       if(int rc = feResidentJacobi(ctx, o, ctx->d_du, &R)) return rc;
     } else {
+      // a zero right-hand side needs no hierarchy
+      if(!ctx->amg)
+        if(int rc = rhsNorm()) return rc;
       const auto s0 = std::chrono::steady_clock::now();
-      if(int rc = feAmgSetup(ctx)) return rc;
+      if(bn != 0.)
+        if(int rc = feAmgSetup(ctx)) return rc;
       setupMs = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - s0).count();
-      if(feAmgNestedUsable(ctx))
+      if(bn != 0. && feAmgNestedUsable(ctx))
         if(int rc = feAmgResidentSolve(ctx, o, ctx->d_du, &R)) return rc;
     }
     if(R.ran) {
@@ -1800,13 +1814,8 @@ int feSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *given, double *du, fe_hip
     }
   }
 
-  hipLaunchKernelGGL(sumSquares, dim3(kGrid), dim3(kTB), 0, ctx->stream, n, ctx->d_rhs, w.part);
-  hipLaunchKernelGGL(finalizeSums, dim3(1), dim3(kTB), 0, ctx->stream, w.part, kGrid, 1, w.res + 8);
-  FE_HIP_TRY(ctx, hipGetLastError());
-  double bb = 0.;
-  FE_HIP_TRY(ctx, hipMemcpyAsync(&bb, w.res + 8, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  FE_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  const double bn = std::sqrt(bb);
+  if(bn < 0.)
+    if(int rc = rhsNorm()) return rc;
   const double target = std::max(o->rtol * bn, o->atol);
   int iters = 0, outer = 0, converged = 0, reason = 0, done = 0, breakdowns = 0;
   double relres = bn > 0. ? 1. : 0.;

@@ -111,3 +111,17 @@ def test_set_up_time_is_reported(resident):
     assert S.get_tuning("resident_ran") == resident
     assert first.ms_setup > 0.3 and first.ms_setup > 5 * second.ms_setup and first.ms_setup < first.ms_solve
     S.close()
+
+
+def test_a_zero_right_hand_side_builds_no_hierarchy():
+    from feng_amd.api import PC_AMG
+    S, _ = _system(4, 24)
+    _, rhs = S.get_system()
+    S.set_system(rhs=np.zeros_like(rhs))
+    r, x = S.solve(pc=PC_AMG, want_du=True)
+    assert r.converged and r.iterations == r.outer_iterations == 0 and r.relres == 0.0 and not x.any()
+    assert r.ms_setup < 0.1 and S.get_tuning("resident_ran") == 0
+    S.set_system(rhs=rhs)
+    r = S.solve(pc=PC_AMG)
+    assert r.converged and r.ms_setup > 0.3 and S.get_tuning("resident_ran") == 1
+    S.close()

@@ -171,6 +171,7 @@ constexpr int kGmAhead = 2;      // steps the host launches ahead of the last po
 constexpr int kGmChunks = 128;   // row chunks of the dot products: partials per vector that every block folds
 constexpr int kGmMaxVec = 128;   // vectors of one cycle (restart + 1 at most)
 constexpr int kGmNorm = 512;     // blocks (norm partials) of the row kernels
+constexpr size_t kGmKeep = (size_t)256 << 20;  // bytes of a workspace kept for the next solve
 
 // Device state of a solve: rotations, the least-squares right-hand side, the
 // last cycle's coefficients, norms.
@@ -596,7 +597,9 @@ struct Gm {
 
 }  // namespace
 
-// Workspace of the GMRES solves of a context, kept between them.
+// Workspace of the GMRES solves of a context, kept between them up to kGmKeep
+// bytes (allocating 50 MB takes longer than a step; above, solves take tens of
+// milliseconds and give (restart + 8) n values back).
 struct FeGmres {
   double *work = nullptr;
   size_t count = 0;
@@ -796,5 +799,10 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
     stats->ms_setup = setupMs;
   }
   if(du) FE_HIP_TRY(ctx, hipMemcpy(du, g.x, sizeof(double) * n, hipMemcpyDeviceToHost));
+  if(W.count * sizeof(double) > kGmKeep) {  // the stream is idle
+    feFree(ctx, W.work);
+    W.work = nullptr;
+    W.count = 0;
+  }
   return FE_STATUS_OK;
 }

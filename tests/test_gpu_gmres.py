@@ -2,6 +2,8 @@
 products, cycle lengths around the 64-vector variant of the projection
 kernels and at the ends of the accepted range, both orthogonalizations,
 against dense solves; the iteration budget and the repeated solve."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -85,4 +87,29 @@ def test_exact_ilu0_application(kind, N):
     t = du @ z / (z @ z)
     # rounding of the solves only: (longest row + levels) units in the last place, amplified by the growth in z
     assert np.linalg.norm(du - t * z) <= 1e-10 * np.linalg.norm(du)
+    S.close()
+
+
+def _free_bytes():
+    """Free device memory, from the HIP runtime the library has loaded."""
+    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64.so" in ln)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_a_large_workspace_is_given_back():
+    """360,000 rows at restart 120: 367 MB during the solve, freed after it; the
+    results of repeated solves do not depend on it."""
+    from feng_amd.api import KSP_GMRES, PC_JACOBI, FN_CONST, Fn, Mesh
+    from feng_amd.problems import diffusion_system
+    S, _ = diffusion_system(Mesh.square(600), 1, 4, Fn(FN_CONST, 1.0), Fn(FN_CONST, -1.0))
+    S.assemble(3)
+    opts = dict(ksp=KSP_GMRES, pc=PC_JACOBI, restart=120, rtol=1e-12, max_iter=20, want_du=True)
+    S.solve(**{**opts, "restart": 2, "max_iter": 2})
+    free = _free_bytes()
+    r0, x0 = S.solve(**opts)
+    assert free - _free_bytes() <= 64 << 20
+    r1, x1 = S.solve(**opts)
+    assert r0.iterations == r1.iterations == 20 and np.array_equal(x0, x1)
     S.close()

@@ -743,7 +743,7 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
     if(!last) outer++;
     if(code >= 2) {  // at the cycle's start
       converged = code == 2;
-      reason = code == 2 ? 2 : -4;
+      reason = code == 2 ? 2 : last ? -3 : -4;
       break;
     }
     if(last) {
@@ -788,7 +788,7 @@ int feSolveGmres(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *du, fe_hi
     double mv[3] = {0., 0., 0.};
     for(size_t q = 0; q < mx.size(); ++q) mv[q % 3] = std::max(mv[q % 3], mx[q]);
     stats->iterations = iters;
-    stats->outer_iterations = outer;
+    stats->outer_iterations = tail[0] == 0. ? 0 : outer;  // no cycle for a zero right-hand side
     stats->converged = converged;
     stats->reason = reason;
     stats->relres_fp64 = tail[0] > 0. ? tail[2] / tail[0] : 0.;

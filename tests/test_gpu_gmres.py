@@ -113,3 +113,17 @@ def test_a_large_workspace_is_given_back():
     r1, x1 = S.solve(**opts)
     assert r0.iterations == r1.iterations == 20 and np.array_equal(x0, x1)
     S.close()
+
+
+def test_what_a_solve_without_iterations_reports():
+    from feng_amd.api import KSP_GMRES, PC_JACOBI
+    S, _, rhs = _system(12)
+    bad = rhs.copy()
+    bad[3] = np.nan
+    # a zero right-hand side starts no cycle; no budget left is -3 whatever the residual, not a number -4
+    for b, max_iter, want in ((0.0 * rhs, 50, (0, 0, True, 2)), (rhs, 0, (0, 0, False, -3)), (bad, 50, (0, 1, False, -4)),
+                              (bad, 0, (0, 0, False, -3))):
+        S.set_system(rhs=b)
+        r = S.solve(ksp=KSP_GMRES, pc=PC_JACOBI, max_iter=max_iter)
+        assert (r.iterations, r.outer_iterations, r.converged, r.reason) == want
+    S.close()

@@ -49,7 +49,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -1143,7 +1142,7 @@ int feAmgResidentSolve(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, double *x, 
   a.wait = resWaitTicks(ctx);
   bool fits = false;
   {
-    std::lock_guard<std::mutex> lock(feResidentMutex(ctx->device));
+    const FeResidentPass pass(ctx, a.G);
     const size_t cells = kSets * a.bufLen;
     hipLaunchKernelGGL(arFill, dim3((unsigned)std::min<size_t>(1024, (cells + 255) / 256)), dim3(256), 0, ctx->stream,
                        cells, a.buf, a.out);

@@ -20,15 +20,35 @@
 // give up the same way, and the host repeats the solve with the
 // launch-per-iteration kernels.
 // All workgroups of a launch must be resident together: the host checks the
-// occupancy and lets one resident launch run per device at a time.
+// occupancy and admits to a device what fits it together (fe_resident_gate.h).
 #pragma once
 
 #include "fe_hip_internal.h"
+#include "fe_resident_gate.h"
 
-#include <mutex>
+// Of a device.
+FeResidentGate &feResidentGate(int device);
 
-// Held from a resident launch to its end (one per device).
-std::mutex &feResidentMutex(int device);
+// Held from a resident launch of G workgroups to its end.
+class FeResidentPass {
+ public:
+  FeResidentPass(fe_hip_ctx *ctx, int G) : gate_(feResidentGate(ctx->device))
+  {
+    int cus = 0;
+    if(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) cus = 0;
+    need_ = feGateNeed(G, cus);
+    // others wait, or are waited for: not inside for this stream's earlier work
+    if(gate_.busy()) (void)hipStreamSynchronize(ctx->stream);
+    gate_.enter(need_, kGateCus);
+  }
+  ~FeResidentPass() { gate_.leave(need_); }
+  FeResidentPass(const FeResidentPass &) = delete;
+  FeResidentPass &operator=(const FeResidentPass &) = delete;
+
+ private:
+  FeResidentGate &gate_;
+  int need_;
+};
 
 namespace fe_res {
 

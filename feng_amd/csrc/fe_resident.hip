@@ -30,7 +30,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -786,10 +785,10 @@ int resBuild(fe_hip_ctx *ctx, FeResident &R)
 
 }  // namespace
 
-std::mutex &feResidentMutex(int device)
+FeResidentGate &feResidentGate(int device)
 {
-  static std::mutex m[64];
-  return m[device & 63];
+  static FeResidentGate g[64];
+  return g[device & 63];
 }
 
 namespace {
@@ -802,7 +801,7 @@ int resRun(fe_hip_ctx *ctx, const fe_hip_solver_opts *o, FeResident &R, unsigned
 {
   bool fits = false;
   {
-    std::lock_guard<std::mutex> lock(feResidentMutex(ctx->device));
+    const FeResidentPass pass(ctx, R.G);
     if(ctx->profiling)
       if(int rc = feTimerMark(ctx, ctx->spmvTimer)) return rc;
     hipLaunchKernelGGL(resFill, dim3((unsigned)std::min<size_t>(1024, (cells + 255) / 256)), dim3(256), 0, ctx->stream,

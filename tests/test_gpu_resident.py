@@ -69,8 +69,11 @@ def test_resident_restarts_from_the_true_residual():
     S.close()
 
 
-def test_resident_two_threads():
-    systems = [_system(1, 90, s)[0] for s in range(2)] + [_system(4, 24, s)[0] for s in range(2)]
+# sizes of which several fit the device together, and ones that need all of it
+@pytest.mark.parametrize("sizes", [[(1, 90), (1, 90), (4, 24), (4, 24)],
+                                   [(1, 20), (1, 40), (4, 12), (4, 30), (1, 500), (4, 60), (1, 64), (4, 16)]])
+def test_resident_threads(sizes):
+    systems = [_system(kind, N, s)[0] for s, (kind, N) in enumerate(sizes)]
     want = [S.solve(rtol=1e-9, want_du=True)[1] for S in systems]
     got = [None] * len(systems)
 

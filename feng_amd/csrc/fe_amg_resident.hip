@@ -1103,6 +1103,7 @@ int launchAr(fe_hip_ctx *ctx, const FeAmgResident &R, const ArArgs &a, bool *fit
 {
   const void *f = (const void *)arSolve<RPT, E>;
   int perCu = 0, cus = 0;
+  std::lock_guard<std::mutex> lock(feResidentGate(ctx->device).launching());
   *fits = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, R.lds) == hipSuccess &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, f, kTB, R.lds) == hipSuccess &&
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) == hipSuccess &&

@@ -729,6 +729,7 @@ int launchRes(fe_hip_ctx *ctx, void (*kernel)(Args), int TB, const FeResident &R
 {
   const void *f = (const void *)kernel;
   int perCu = 0, cus = 0;
+  std::lock_guard<std::mutex> lock(feResidentGate(ctx->device).launching());
   *fits = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, f, TB, lds) == hipSuccess &&
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) == hipSuccess &&

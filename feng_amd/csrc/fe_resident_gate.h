@@ -33,9 +33,12 @@ class FeResidentGate {
     std::lock_guard<std::mutex> lock(m_);
     return used_ > 0 || admitted_ != arrived_;
   }
+  // Held while a kernel's LDS limit, which all threads share, is set and the
+  // kernel launched with it.
+  std::mutex &launching() { return launch_; }
 
  private:
-  std::mutex m_;
+  std::mutex m_, launch_;
   std::condition_variable cv_;
   int used_ = 0;
   unsigned long long arrived_ = 0, admitted_ = 0;

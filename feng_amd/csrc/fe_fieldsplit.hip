@@ -283,6 +283,7 @@ int fsPattern(fe_hip_ctx *ctx)
   sub->amgLanes = ctx->amgLanes;
   sub->amgPadTiles = ctx->amgPadTiles;
   sub->amgKernel = ctx->amgKernel;
+  sub->amgFuse = 0;  // its barriers are checked after a synchronization, which an application here does without
   sub->pcValues32 = ctx->pcValues32;
   return FE_STATUS_OK;
 }

@@ -458,8 +458,9 @@ int feAmgPcgVcycle(fe_hip_ctx *ctx, const double *r, double *z);
 // The V-cycle in the nested order without copies or synchronization, for
 // callers that keep their own maps: the device permutation (nested row ->
 // row), the right-hand side it reads and the result it writes, and its
-// launches (feAmgPcgPrepare first; the fused coarse launch of amg_fuse, whose
-// barriers are checked after a synchronization, is not taken here).
+// launches (feAmgPcgPrepare first; with amg_fuse the caller has to check the
+// fused coarse launch's barriers after a synchronization, as feAmgPcgVcycle
+// does).
 void feAmgPcgNested(const fe_hip_ctx *ctx, const int **perm, double **rhs, const double **z);
 int feAmgPcgVcycleLaunch(fe_hip_ctx *ctx);
 

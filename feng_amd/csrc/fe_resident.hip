@@ -22,10 +22,12 @@
 // 16.9 -> 5.5, 64^3 24.0 -> 6.2 us.  What is left is the trip of a stored word
 // to another workgroup's poll (about 1.5 us), the LDS gathers and the barriers.
 //
-// The rule (resUsable): one row a thread on the CUs of the device (n <= 1024 x
+// The rule (resBuild): one row a thread on the CUs of the device (n <= 1024 x
 // CUs, 262,144 on 256), rows of at most 24 entries (48 + 12 registers), and
 // the rows of other workgroups that one gathers have to fit the LDS.  Larger
 // systems are bound by the matrix traffic, which the tiled kernels stream.
+// resSplit: rows of at most 16 entries above 512 x CUs rows (131,072), where
+// workgroups have 1024 threads and no registers for longer ones.
 #include "fe_resident.h"
 
 #include <algorithm>

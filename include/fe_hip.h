@@ -100,8 +100,10 @@ typedef struct {
 
 #define FE_PREC_FP64 0    /* FP64 Krylov */
 /* FP32 inner Krylov + FP64 iterative refinement; CG runs in FP64 instead where
- * that is faster: solves that fit one launch (about 260,000 rows of at most 24
- * entries), multigrid-PCG up to 700,000 rows */
+ * that is faster: Jacobi and split solves that fit one launch (on 256 CUs
+ * 262,144 rows of at most 24 entries; the split preconditioners above 131,072
+ * rows of at most 16), multigrid-PCG up to 700,000 rows (tuning key
+ * "amg_fp32_rows") */
 #define FE_PREC_FP32_IR 1
 
 typedef struct {

@@ -11,14 +11,17 @@ One step = zero + assemble (the one-launch row-gather assembly of every
 element term into the device CSR and RHS, with the FP32 copy of the values
 on the FP32 paths) + solve, inputs already resident in HBM.  Paths:
   plain   : FP64 Jacobi-PCG (pipelined, one kernel/iteration)
-  fast    : FP32 Jacobi-PCG inner solves, FP64 iterative refinement
+  fast    : the same at FE_PREC_FP32_IR: the FP64 iteration where the solve
+            runs as one launch (n = 250,047 does), else FP32 Jacobi-PCG inner
+            solves with FP64 iterative refinement
   learned : as fast, with the learned IC(0)-pattern split preconditioner
             (weights from feng_amd/weights/, skipped when absent)
   learned64 : FP64 split PCG with the learned preconditioner
   ic0     : FP64 split IC(0)-pattern PCG (the learned path without the net)
   amg     : FP64 PCG preconditioned by the aggregation-multigrid V-cycle over
             the nested ordering (FP32 level values)
-  amg32   : the same in FP32, FP64 refinement by residual replacement
+  amg32   : the same at FE_PREC_FP32_IR: FP64 up to 700,000 rows, above in
+            FP32 with FP64 refinement by residual replacement
 `value` is the DOF/s of the fastest non-plain path (named in config.path);
 every path is reported in config.paths, with its speed-up over plain.
 
@@ -103,18 +106,31 @@ ITER_KERNEL = {
     "amg": ("pcgDown0<double, float> (level-0 CG update + smoothing + restriction)", 8),
     "amg32": ("pcgDown0<float, float> (level-0 CG update + smoothing + restriction)", 4),
 }
-# Kernels that run every iteration of a solve in one launch (matrix and vectors
-# stay on chip, systems of up to about 260,000 rows): timed figures and bytes
-# are per iteration, and the bytes are what a launch per iteration would move.
+# Kernels that run every iteration of a solve in one launch: timed figures are
+# the launch's time over its iterations, bytes are those of a launch.
 RESIDENT_KERNEL = {
-    "plain": "resJacobi (all iterations in one launch; per iteration)",
-    "fast": "resJacobi (all iterations in one launch; per iteration)",
-    "learned": "resSplit (all iterations in one launch; per iteration)",
-    "learned64": "resSplit (all iterations in one launch; per iteration)",
-    "ic0": "resSplit (all iterations in one launch; per iteration)",
-    "amg": "arSolve (all iterations in one launch; per iteration)",
-    "amg32": "arSolve (all iterations in one launch; per iteration)",
+    "plain": "resJacobi (all iterations in one launch)",
+    "fast": "resJacobi (all iterations in one launch)",
+    "learned": "resSplit (all iterations in one launch)",
+    "learned64": "resSplit (all iterations in one launch)",
+    "ic0": "resSplit (all iterations in one launch)",
+    "amg": "arSolve (all iterations in one launch)",
+    "amg32": "arSolve (all iterations in one launch)",
 }
+
+
+def one_launch_bytes(pc, rows, nnzs):
+    """Bytes a one-launch solve cannot do without: the matrix once (FP64 values,
+    16-bit positions), the factor's FP32 values once or the levels' (FP32
+    values, 16-bit positions), right-hand side and solution.  The words that
+    workgroups exchange come on top, in every iteration; they bound it by
+    their latency."""
+    b = 10 * nnzs[0] + 4 * rows[0] + 16 * rows[0]
+    if pc == "amg":
+        b += sum(6 * z + 8 * r for r, z in zip(rows[1:], nnzs[1:]))
+    elif pc != "jacobi":
+        b += 4 * nnzs[0]
+    return b
 
 
 def iter_bytes(s, n, nnz):
@@ -179,7 +195,8 @@ def run_step(S, path, rtol, profile=False):
     spmv_ms, launches = S.kernel_stats(0)
     iter_ms, _ = S.kernel_stats(2)
     return dict(wall_s=wall, asm_ms=asm_ms, solve_ms=r.ms_solve, iters=r.iterations, outer=r.outer_iterations,
-                relres=r.relres, converged=r.converged, spmv_ms=spmv_ms, spmv_launches=launches, iter_ms=iter_ms)
+                relres=r.relres, converged=r.converged, spmv_ms=spmv_ms, spmv_launches=launches, iter_ms=iter_ms,
+                one_launch=bool(S.get_tuning("resident_ran")))
 
 
 def cpu_baseline(m, k, num, rtol, budget_s=25.0):
@@ -700,8 +717,9 @@ def main():
     v32 = S.get_system32()
     fp32_err = float(np.abs(v32.astype(np.float64) - v64).max() / np.abs(v64).max())
     fast_paths = [p for p in ("fast", "learned", "learned64", "amg", "amg32") if p in res] or ["plain"]
-    if n <= 700000 and "amg" in res and "amg32" in fast_paths:
-        fast_paths.remove("amg32")  # the same FP64 iteration
+    amg32_is_64 = n <= S.get_tuning("amg_fp32_rows")  # the same FP64 iteration
+    if amg32_is_64 and "amg" in res and "amg32" in fast_paths:
+        fast_paths.remove("amg32")
     best = min(fast_paths, key=lambda p: res[p]["ms"])
     B = res[best]
     plain = res["plain"]
@@ -709,24 +727,25 @@ def main():
     # roofline of the dominant kernel of the reported path: one PCG iteration
     # launch.  Algorithmic bytes per iteration (minimal unfused PCG-Jacobi):
     # values s nnz + column ids 4 nnz + row pointers 4 (n+1) + 18 vector
-    # passes of s n.  FP32 inner solve: s = 4.
+    # passes of s n.  FP32 inner solve: s = 4.  A solve that ran as one launch
+    # keeps matrix and vectors on chip: its bytes are those of the launch.
     kern_ms = B["prof"]["spmv_ms"]
     kname, sz = ITER_KERNEL[best]
-    # one launch for all iterations: both timers hold its time over the iterations
-    resident = best in RESIDENT_KERNEL and kern_ms and kern_ms == B["prof"]["iter_ms"]
-    if best == "amg32" and n <= 700000:  # the FP64 iteration
+    resident = B["prof"]["one_launch"]
+    if best == "amg32" and amg32_is_64:
         kname, sz = ITER_KERNEL["amg"]
-    if PATHS[best][1] != "amg" and n <= 262144:
-        resident = True
+    per_iter = None
     if resident:
         kname, sz = RESIDENT_KERNEL[best], 8
-    per_iter = None
-    if PATHS[best][1] == "amg":
+        kern_ms *= B["prof"]["iters"]
+        extra = B.get("extra", {"amg_rows": [n], "amg_nnz": [nnz]})
+        alg_bytes = one_launch_bytes(PATHS[best][1], extra["amg_rows"], extra["amg_nnz"])
+    elif PATHS[best][1] == "amg":
         # dominant kernel by profiled time: the level-0 restriction pcgDown0, or all of the iteration
         rows_l, nnz_l = B["extra"]["amg_rows"], B["extra"]["amg_nnz"]
         v = 4  # level values FP32 (pc_values32 = 1)
         it_bytes = mg_iter_bytes(sz, v, 8 if sz == 8 else 4, rows_l, nnz_l)
-        alg_bytes = it_bytes if resident else mg_down0_bytes(sz, v, n, nnz, rows_l[1])
+        alg_bytes = mg_down0_bytes(sz, v, n, nnz, rows_l[1])
         it_ms = B["prof"]["iter_ms"]
         per_iter = {"alg_bytes": it_bytes, "avg_ms": it_ms,
                     "frac": it_bytes / (it_ms * 1e-3) / 1e9 / HBM_PEAK_GBS if it_ms else None}
@@ -738,8 +757,8 @@ def main():
     b_asm = asm_bytes(m.E, m.V, n, nnz)
     asm_ms = float(np.mean([x["asm_ms"] for x in B["steps"]]))
     per_step = None
-    if per_iter:
-        step_bytes = b_asm + per_iter["alg_bytes"] * B["last"]["iters"]
+    if per_iter or resident:
+        step_bytes = b_asm + (alg_bytes if resident else per_iter["alg_bytes"] * B["last"]["iters"])
         per_step = {"alg_bytes": step_bytes, "ms": B["ms"],
                     "frac": step_bytes / (B["ms"] * 1e-3) / 1e9 / HBM_PEAK_GBS}
 
@@ -769,6 +788,7 @@ def main():
                 "relres": r["last"]["relres"], "asm_ms": float(np.mean([x["asm_ms"] for x in r["steps"]])),
                 "solve_ms": float(np.mean([x["solve_ms"] for x in r["steps"]])),
                 "iter_kernel_ms": r["prof"]["spmv_ms"], "iteration_ms": r["prof"]["iter_ms"] or None,
+                "one_launch": r["prof"]["one_launch"],
                 **r.get("extra", {})}
 
     out = {
@@ -786,8 +806,9 @@ def main():
         "data": "synthetic (seeded GRF coefficient on a generated Kuhn-tet cube)",
         "config": {"workload": f"P1 tet diffusion, unit cube {args.N}^3 x6 Kuhn tets, k=exp(GRF l=0.1 s=1.5), "
                                f"PCG to FP64 rel-res 1e-8", "n": n, "nnz": nnz, "elements": m.E,
-                   "path": {"fast": "FP32 Jacobi-PCG + FP64 iterative refinement",
-                            "learned": "FP32 learned-IC(0) split PCG + FP64 iterative refinement",
+                   "path": {"fast": "Jacobi-PCG at FE_PREC_FP32_IR: FP64 in one launch, or FP32 with FP64 refinement",
+                            "learned": "learned-IC(0) split PCG at FE_PREC_FP32_IR: FP64 in one launch, or FP32 with "
+                                       "FP64 refinement",
                             "learned64": "FP64 learned-IC(0) split PCG",
                             "amg": "FP64 PCG with the aggregation-multigrid V-cycle (FP32 level values)",
                             "amg32": "PCG with the aggregation-multigrid V-cycle at FE_PREC_FP32_IR: FP64 up to "
@@ -796,8 +817,10 @@ def main():
                    "paths": {p: {**summary(p), "speedup_vs_plain_fp64": plain["ms"] / res[p]["ms"]} for p in res},
                    "speedup_vs_plain_fp64": plain["ms"] / B["ms"],
                    "fp32_value_error_vs_fp64": fp32_err,
-                   "plain_iter_roofline_frac": p_alg / (p_kern * 1e-3) / 1e9 / HBM_PEAK_GBS if p_kern else None},
-        "roofline": {"bound": "hbm", "kernel": kname, "achieved": achieved, "peak": HBM_PEAK_GBS,
+                   # a launch per iteration only: in one launch the matrix stays on chip
+                   "plain_iter_roofline_frac": p_alg / (p_kern * 1e-3) / 1e9 / HBM_PEAK_GBS
+                   if p_kern and not plain["prof"]["one_launch"] else None},
+        "roofline": {"bound": "latency of the exchanges between workgroups" if resident else "hbm", "kernel": kname, "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": TRAFFIC.get(kname),
                      "avg_launch_ms": kern_ms, "alg_bytes_per_launch": alg_bytes,
                      "per_iteration": per_iter, "per_step": per_step,

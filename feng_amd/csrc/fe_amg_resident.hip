@@ -113,7 +113,7 @@ struct ArArgs {
   double *maxima;
   double rtol, atol, dtol, oc;
   int maxit;
-  long long wait;  // ticks
+  int wait;  // ticks
 };
 
 // LDS positions of the columns of a workgroup's rows (see fe_resident.hip):
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
   extern __shared__ __align__(16) unsigned char lds[];
   constexpr int kHeld = RPT == 1 ? 2 : 4;
   __shared__ double wsum[3][4], psum[3][kTB / 64];
-  __shared__ int gaveUp;
+  __shared__ int gaveUp, wait;
   __shared__ int4 info[kMaxDist + 1];  // per level: first own row, own rows, gathered rows
   const int wg = blockIdx.x, t = threadIdx.x, G = a.G, B = a.B;
   const ArDist &L0 = a.lv[0];
@@ -373,7 +373,10 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
   const int hc0 = L0.hcnt[wg];
   const int *hcol0 = L0.hcol + (size_t)wg * L0.hcap;
   const int pb = a.partBase[wg], pc = a.partBase[wg + 1] - pb, pf = a.partFirst[wg];
-  if(t == 0) gaveUp = 0;
+  if(t == 0) {
+    gaveUp = 0;
+    wait = a.wait;
+  }
   // --- what stays for the whole solve
   for(int c = t; c < a.blk.bytes / 16; c += kTB) ((uint4 *)(lds + a.blk.lImg))[c] = ((const uint4 *)a.img)[c];
   for(int l = 0; l < B; ++l) {
@@ -467,14 +470,14 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
     }
 #pragma unroll
     for(int k = 0; k < kHeld; ++k) at[kS + k] = hcl[k] >= 0 ? o + hcl[k] : -1;
-    bool ok = resPoll<kS + kHeld>(buf, at, pv, a.wait);
+    bool ok = resPoll<kS + kHeld>(buf, at, pv, wait);
 #pragma unroll
     for(int k = 0; k < kHeld; ++k)
       if(hcl[k] >= 0) reg[L0.rows + t + k * kTB] = __longlong_as_double((long long)pv[kS + k]);
     for(int h = t + kHeld * kTB; h < hc0 && ok; h += kTB) {
       const int a1[1] = {o + hcol0[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1, a.wait);
+      ok = resPoll<1>(buf, a1, v1, wait);
       reg[L0.rows + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;
@@ -553,7 +556,7 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
     for(int h = t; h < hc && ok; h += kTB) {
       const int a1[1] = {o + hcol[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1, a.wait);
+      ok = resPoll<1>(buf, a1, v1, wait);
       reg[L.rows + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;
@@ -724,7 +727,7 @@ __global__ __launch_bounds__(kTB) void arSolve(ArArgs a)
       for(int i = t; i < a.parts && ok; i += 2 * kTB) {
         const int a2[2] = {a.oParts + i, i + kTB < a.parts ? a.oParts + i + kTB : -1};
         unsigned long long v2[2];
-        ok = resPoll<2>(buf, a2, v2, a.wait);
+        ok = resPoll<2>(buf, a2, v2, wait);
         parts[i] = __longlong_as_double((long long)v2[0]);
         if(i + kTB < a.parts) parts[i + kTB] = __longlong_as_double((long long)v2[1]);
       }

@@ -78,10 +78,7 @@ __device__ __forceinline__ void resStoresDone() { asm volatile("s_waitcnt vmcnt(
 
 // The longest wait of a launch, in ticks of the 100 MHz counter; 0 us: no wait
 // at all, give up on the first value that has not arrived.
-inline long long resWaitTicks(const fe_hip_ctx *ctx)
-{
-  return ctx->residentWaitUs > 0 ? 100ll * ctx->residentWaitUs : -1;
-}
+inline int resWaitTicks(const fe_hip_ctx *ctx) { return ctx->residentWaitUs > 0 ? 100 * ctx->residentWaitUs : -1; }
 
 // A solve that the iteration limit of a launch has cut short of its own budget:
 // the launches per iteration repeat it.
@@ -91,10 +88,11 @@ inline bool resCutShort(const fe_hip_ctx *ctx, const fe_hip_solver_opts *o, int 
 }
 
 // Polls the K slots base[idx[k]] (idx < 0: none) until all have arrived; false
-// when the time is up.  The loads of a round are issued together.
+// when the time (ticks, in LDS: scalar registers are short) is up.  The loads
+// of a round are issued together.
 template <int K>
 __device__ __forceinline__ bool resPoll(const unsigned long long *base, const int (&idx)[K], unsigned long long (&v)[K],
-                                        long long ticks)
+                                        const int &ticks)
 {
 #pragma unroll
   for(int k = 0; k < K; ++k) v[k] = idx[k] >= 0 ? resLoad(base + (unsigned)idx[k]) : 0ull;

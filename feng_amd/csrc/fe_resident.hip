@@ -78,7 +78,7 @@ struct ResArgs {
   int maxit;
   int refine;      // FE_PREC_FP32_IR: the targets are tested before the first iteration too, with a bound on
                    // the restarts, as in that loop
-  long long wait;  // ticks
+  int wait;  // ticks
 };
 
 // LDS positions of a workgroup's entries: own rows first, then the other
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
   constexpr int kSums = kSplit ? 0 : 3, kHeld = kSplit ? 6 : 3, kPoll = kSums + kHeld;
   extern __shared__ double lds[];           // two regions of own + gathered values
   __shared__ double wsum[3][16], psum[3][TB / 64];
-  __shared__ int gaveUp;
+  __shared__ int gaveUp, wait, refine;
   const int wg = blockIdx.x, t = threadIdx.x, G = a.G, RW = a.RW, stride = RW + a.H;
   const int row = wg * RW + t;
   const bool own = t < RW && row < a.n;
@@ -205,7 +205,11 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
   const int hc = a.hcnt[wg];
   const int *hcol = a.hcol + (size_t)wg * a.hcap;
   const int sumThreads = (G + 63) & ~63, h0 = kSplit ? t - sumThreads : t, hStep = kSplit ? TB - sumThreads : TB;
-  if(t == 0) gaveUp = 0;
+  if(t == 0) {
+    gaveUp = 0;
+    wait = a.wait;
+    refine = a.refine;
+  }
   // entries, 1 / a_ii, vectors
   double v[E];
   unsigned ix[E / 2];
@@ -271,14 +275,14 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
 #pragma unroll
       for(int k = 0; k < 3; ++k)
         if(!kSplit || t < sumThreads) at[k] = t < G ? a.n + k * G + t : -1;
-      bool ok = resPoll<kPoll>(buf, at, pv, a.wait);
+      bool ok = resPoll<kPoll>(buf, at, pv, wait);
 #pragma unroll
       for(int k = 0; k < kHeld; ++k)
         if(hcl[k] >= 0) reg[RW + h0 + k * hStep] = __longlong_as_double((long long)pv[kSums + k]);
       for(int h = h0 + kHeld * hStep; h0 >= 0 && h < hc && ok; h += hStep) {
         const int a1[1] = {hcol[h]};
         unsigned long long v1[1];
-        ok = resPoll<1>(buf, a1, v1, a.wait);
+        ok = resPoll<1>(buf, a1, v1, wait);
         reg[RW + h] = __longlong_as_double((long long)v1[0]);
       }
       if(t < G) {
@@ -344,22 +348,22 @@ __global__ __launch_bounds__(TB) void resJacobi(ResArgs a)
         target = resUniform(fmax(a.rtol * bn, a.atol));
         tol2 = resUniform(target * target * 0.25);
         if(bn == 0.) reason = 2;
-        else if(a.refine && rn <= target) reason = 2;
-        else if(a.refine && a.maxit <= 0) reason = -3;
+        else if(refine && rn <= target) reason = 2;
+        else if(refine && a.maxit <= 0) reason = -3;
         if(reason) break;
       } else {
         if(rn <= target) reason = 2;
         else if(code == 4 || !(rn == rn)) reason = -9;
-        else if(it >= a.maxit && !a.refine) reason = -3;
+        else if(it >= a.maxit && !refine) reason = -3;
         else if(rn / bn > a.dtol) reason = -4;
         else if(code == 3 && ++breakdowns > 20) reason = -3;
-        else if(a.refine && outer >= kResOuter) reason = kResLimit;
+        else if(refine && outer >= kResOuter) reason = kResLimit;
         else if(it >= a.maxit) reason = -3;
         if(reason) break;
         // again from the true residual: after a breakdown, or when the
         // recursive residual met a target the true one has not (aim lower; the
         // bounded restarts of a refined solve keep the target)
-        if(code != 3 && !a.refine) tol2 = resUniform(0.01 * tol2);
+        if(code != 3 && !refine) tol2 = resUniform(0.01 * tol2);
         code = 0;
       }
       s = z = p = 0.;
@@ -476,7 +480,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
   constexpr int kHeld = TB == 512 ? 3 : 2;
   extern __shared__ double lds[];           // two regions of own + gathered values
   __shared__ double wsum[3][4], psum[3][TB / 64];
-  __shared__ int gaveUp, below;
+  __shared__ int gaveUp, wait, below;
   const int wg = blockIdx.x, t = threadIdx.x, G = a.G, RW = a.RW, stride = RW + a.H;
   const int r0 = wg * RW, row = r0 + t;
   const bool own = t < RW && row < a.n;
@@ -486,6 +490,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
   const int *hcol = a.hcol + (size_t)wg * a.hcap;
   if(t == 0) {
     gaveUp = 0;
+    wait = a.wait;
     below = 0;
   }
   for(int q = t; q < 2 * stride; q += TB) lds[q] = 0.;  // a factor reads only the columns of its half
@@ -560,7 +565,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
       const int h = t + k * TB;
       at[kS + k] = h >= h0 && h < h1 ? o + hcl[k] : -1;
     }
-    bool ok = resPoll<kS + kHeld>(buf, at, pv, a.wait);
+    bool ok = resPoll<kS + kHeld>(buf, at, pv, wait);
 #pragma unroll
     for(int k = 0; k < kHeld; ++k)
       if(at[kS + k] >= 0) reg[RW + t + k * TB] = __longlong_as_double((long long)pv[kS + k]);
@@ -568,7 +573,7 @@ __global__ __launch_bounds__(TB) void resSplit(SplitArgs sa)
       if(h < h0) continue;
       const int a1[1] = {o + hcol[h]};
       unsigned long long v1[1];
-      ok = resPoll<1>(buf, a1, v1, a.wait);
+      ok = resPoll<1>(buf, a1, v1, wait);
       reg[RW + h] = __longlong_as_double((long long)v1[0]);
     }
     if(!ok) gaveUp = 1;

@@ -60,6 +60,9 @@ TRAFFIC = {  # HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE (cube
     "pcgDown0<double, float> (level-0 CG update + smoothing + restriction)": 76.2e6,
     "pcgDown0<float, float> (level-0 CG update + smoothing + restriction)": 53.0e6,
     "asmGather<double, 4, 3, 16>": 370.5e6,
+    "resJacobi (all iterations in one launch)": 3558e6,
+    "resSplit (all iterations in one launch)": 16323e6,
+    "arSolve (all iterations in one launch)": 2449e6,
     # the batched workload's level-0 prolongation product over the whole level
     # (draw_problems(256, 1) as one system): profiles/batched256_hbm_traffic.md
     "amgUp<double, float, 4, 256, true>": 2012.9e6,

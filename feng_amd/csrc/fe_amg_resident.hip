@@ -24,9 +24,9 @@
 //       p = z + beta p, q = A z + beta q, a = A w + beta a (= A l1 q);
 //       x += alpha p, r -= alpha q, A u -= alpha a for u = l1 r
 //   y:  z = y + l1 (r - A y)
-// What bounds an iteration is the chain of exchanges (1.1 to 3.5 us for the
-// neighbours' values, 3.2 to 6 us for the sums) and, on the largest matrices,
-// the single-workgroup levels (3.5 us at 190 rows, 12 us at 688), not bytes.
+// What bounds an iteration is the chain of exchanges (1.3 to 3.3 us for the
+// neighbours' values, 3.3 to 6.3 us for the sums) and, on the largest matrices,
+// the single-workgroup levels (3.6 us at 190 rows, 11.6 us at 688), not bytes.
 // Solve with numeric set-up, launch-per-level -> here: 21^3 1.43 -> 0.62 ms,
 // 37^3 2.6 -> 1.15 ms, 64^3 (250,047 unknowns) 4.8 -> 2.38 ms.  Only rows that
 // another workgroup gathers are stored to the exchange buffer: the write-through
@@ -39,9 +39,10 @@
 // complete.
 //
 // The rule (arBuild): two rows a thread of the device (at most 1024 a
-// workgroup, cut at level B - 1 rows), level-0 rows of at most 24 entries, FP64
-// vectors with FP32 level values, and the LDS plan has to fit; otherwise the
-// launch-per-level kernels run.  512 threads leave 256 registers to each; 1024
+// workgroup, cut at level B - 1 rows: 249,001 P1 triangle unknowns fit, 261,121
+// do not), level-0 rows of at most 24 entries, FP64 vectors with FP32 level
+// values, and the LDS plan has to fit; otherwise the launch-per-level kernels
+// run.  512 threads leave 256 registers to each; 1024
 // threads of one row spilled (64 registers more for what does not depend on the
 // row): 3.6 instead of 1.3 us for a product with its resets at 21^3.
 #include "fe_resident.h"
